@@ -233,21 +233,26 @@ static int get_twiddles(hh_context *c, int N, int f32, void **out) {
     return HH_OK;
 }
 
-// S[n][k] = sqrt(2/(N+1)) sin(pi (n+1)(k+1)/(N+1)), exact integer reduction
+// Tables of the dense DST, from sqrt(2/(N+1)) sin(pi q/(N+1)) with the angle
+// reduced exactly in integers, q = (n+1)(k+1) mod 2(N+1): its odd outputs
+// k = 2c and its even ones k = 2c+1 on the first half of the line, each padded
+// to half_dst_rows x half_dst_cols; the middle point of an odd N meets itself
+// in x_j + x_{M-j} and enters at half weight.
 static int get_dst_matrix(hh_context *c, int N, int f32, void **out) {
     auto &m = f32 ? c->S32 : c->S64;
     auto it = m.find(N);
     if (it != m.end()) { *out = it->second; return HH_OK; }
-    std::vector<double> S((size_t)N * N);
-    long M2 = 2L * (N + 1);
-    double s = std::sqrt(2.0 / (N + 1));
-    for (long n = 0; n < N; n++)
-        for (long k = 0; k < N; k++) {
-            long q = ((n + 1) * (k + 1)) % M2;
-            S[n * N + k] = s * (double)sinl(3.14159265358979323846264338327950288L * (long double)q / (long double)(N + 1));
-        }
+    const long M2 = 2L * (N + 1), HP = hh::half_dst_rows(N), WP = hh::half_dst_cols(N), H = (N + 1) / 2;
+    const double s = std::sqrt(2.0 / (N + 1));
+    std::vector<double> sine(M2), S((size_t)2 * HP * WP, 0.0);
+    for (long q = 0; q < M2; q++)
+        sine[q] = s * (double)sinl(3.14159265358979323846264338327950288L * (long double)q / (long double)(N + 1));
+    for (int par = 0; par < 2; par++)
+        for (long n = 0; n < (par == 0 ? H : N / 2); n++)
+            for (long k = par; k < N; k += 2)
+                S[(par * HP + n) * WP + k / 2] = sine[((n + 1) * (k + 1)) % M2] * (2 * n + 1 == N ? 0.5 : 1.0);
     void *d = nullptr;
-    size_t bytes = (size_t)N * N * (f32 ? 4 : 8);
+    size_t bytes = S.size() * (f32 ? 4 : 8);
     int rc = dev_alloc(c, &d, bytes);
     if (rc) return rc;
     if (f32) {

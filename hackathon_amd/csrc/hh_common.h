@@ -60,6 +60,19 @@ template <typename T> HH_DEV T cabs2(C2<T> z) { return z.x * z.x + z.y * z.y; }
 
 template <typename To, typename Ti> HH_DEV C2<To> cconv(C2<Ti> z) { return mk<To>((To)z.x, (To)z.y); }
 
+// Store of one output element: out = X, or out += acc X for an FP64 output
+// with acc != 0 (the refinement update folded into the last pass).
+template <typename To, typename T> HH_DEV void put_out(C2<To> *o, C2<T> v, double acc) {
+    if constexpr (sizeof(To) == 8) {
+        if (acc != 0) {
+            const C2<double> u = *o;
+            *o = mk<double>(u.x + acc * (double)v.x, u.y + acc * (double)v.y);
+            return;
+        }
+    }
+    *o = cconv<To, T>(v);
+}
+
 // Bounds of the kernels: maximum system length handled by one tridiagonal
 // block and maximum FFT length.
 #define HH_FFT_LMAX 8192

@@ -42,14 +42,24 @@ struct Lines {
     double acc = 0;
 };
 
+// Tables of the dense DST: two matrices (odd outputs, then even ones) of
+// half_dst_rows x half_dst_cols, zero outside ceil(N/2) x ceil(N/2) and
+// floor(N/2) x floor(N/2); padded so that no tile of the kernel is cut.
+constexpr int HH_DENSE_HP = 64, HH_DENSE_WP = 32;
+__host__ __device__ inline int half_dst_rows(int N) { return ((N + 1) / 2 + HH_DENSE_HP - 1) / HH_DENSE_HP * HH_DENSE_HP; }
+__host__ __device__ inline int half_dst_cols(int N) { return ((N + 1) / 2 + HH_DENSE_WP - 1) / HH_DENSE_WP * HH_DENSE_WP; }
+
 bool fft_supported(int N);  // N+1 a power of two, 2(N+1) <= HH_FFT_LMAX
 
 // Orthonormal DST-I of every line.  FFT path (in == out allowed) when
 // fft_supported(N), else the dense-matrix path (in != out required).
 // tw: device twiddle table e^{-2 pi i q/L}, L = 2(N+1), in the compute type.
-// S: device DST matrix (N*N, compute type) for the dense path.
+// S: device tables of the dense path in the compute type (the pair above).
 hipError_t launch_dst(const Lines &ln, DstTypes ty, const void *in, void *out,
                       const void *tw, const void *S, hipStream_t st);
+// The dense path alone (element types 0 = double, 1 = float).
+hipError_t launch_dense(const Lines &ln, int algo, int ti, int tc, int to, const void *in, void *out, const void *S,
+                        hipStream_t st);
 
 // Per-mode tridiagonal solves of the Helmholtz operator along the last axis.
 struct TriHelm {
