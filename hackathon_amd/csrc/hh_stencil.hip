@@ -288,11 +288,14 @@ hipError_t launch_rhs3d(const Rhs3D &r, void *F, hipStream_t st) {
 // marches along the last axis over a chunk of rows (2D) or layers (3D),
 // keeping the 3 x 3 (x 3) neighbourhood in registers so that every value of
 // u is loaded about once per thread row; the coefficient row of a step is
-// the same for the whole block.  The sums keep the order of the reference.
-constexpr int RES_ROWS = 8;   // rows (2D) or layers (3D) per thread
+// the same for the whole block and comes through scalar loads (__restrict__: the
+// result never overlaps the table); as vector loads each row's coefficients were
+// waited for behind the row's own.  The sums keep the order of the reference.
+// 64 x 1023^2: 689 -> 599 us (5.4 TB/s), 8 x 1023^2: 93 -> 74 us.
+constexpr int RES_ROWS = 4;   // rows per thread in 2D (8 rows: 618 and 79 us; 16: 663 and 92)
 
 template <typename To>
-__global__ __launch_bounds__(256) void k_residual2d(int Nx, int Ny, int nchunk, const z2 *coef, int nop, const z2 *u,
+__global__ __launch_bounds__(256) void k_residual2d(int Nx, int Ny, int nchunk, const z2 *__restrict__ coef, int nop, const z2 *u,
                                                     const z2 *F, C2<To> *res, int b0) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     const int j0 = blockIdx.y * RES_ROWS;
@@ -334,11 +337,17 @@ __global__ __launch_bounds__(256) void k_residual2d(int Nx, int Ny, int nchunk, 
 // each of its three layers, the four sums the stencil weights.  The loads are software-
 // pipelined: a step stores the layer fetched during the previous step and
 // issues the fetch of the next one (and of the next F value) before its
-// barrier, so HBM latency is not paid once per layer.
-constexpr int RX = 64, RY = 8, RZ = 16;
+// barrier, so HBM latency is not paid once per layer.  The coefficients come
+// through scalar loads (__restrict__: the result never overlaps the table): as
+// vector loads they sat behind the prefetches in the in-order load counter, and
+// every step waited for the next layer it had just asked for.  255^3: 242 ->
+// 165 us (4.8 TB/s), 127 x 255 x 200: 105 -> 71 us; two and three layers ahead
+// measured the same.  Tiles are 64 points wide, 32 where that covers Nx with
+// fewer idle lanes (200^3: 89 against 95 us; 255^3: 178 against 168).
+constexpr int RY = 8, RZ = 16;
 
-template <typename To>
-__global__ __launch_bounds__(RX * RY) void k_residual3d(int Nx, int Ny, int Nz, int nchunk, const z2 *coef, int nop,
+template <typename To, int RX>
+__global__ __launch_bounds__(RX * RY) void k_residual3d(int Nx, int Ny, int Nz, int nchunk, const z2 *__restrict__ coef, int nop,
                                                        const z2 *u, const z2 *F, C2<To> *res, int b0) {
     constexpr int HX = RX + 2, HY = RY + 2, HE = HX * HY, NT = RX * RY;
     static_assert(HE <= 2 * NT, "a layer tile with halo takes at most two loads per thread");
@@ -360,17 +369,20 @@ __global__ __launch_bounds__(RX * RY) void k_residual3d(int Nx, int Ny, int Nz, 
         in = ll >= 0 && ll < Nz && ii >= 0 && ii < Nx && jj >= 0 && jj < Ny;
         return in ? ii + (long)jj * Nx + (long)ll * Nxy : 0;
     };
-    z2 n0, n1;   // the next layer's elements, in flight during a step
+    z2 n0, n1, fn;   // the next layer's elements and right-hand side, in flight during a step
+    auto zsel = [](bool c, z2 v) { return mk<double>(c ? v.x : 0.0, c ? v.y : 0.0); };
     auto fetch = [&](int ll) {
         bool in0, in1;
         const long s0 = src(tid, ll, in0), s1 = src(has1 ? e1 : tid, ll, in1);
-        const z2 v0 = ub[s0], v1 = ub[s1];
-        n0 = in0 ? v0 : zr(0.0);
-        n1 = in1 ? v1 : zr(0.0);
+        n0 = ub[s0];
+        n1 = ub[s1];
     };
-    auto stash = [&](int slot) {
-        lay[slot][tid] = n0;
-        if (has1) lay[slot][e1] = n1;
+    auto stash = [&](int slot, int ll) {
+        bool in0, in1;
+        src(tid, ll, in0);
+        src(has1 ? e1 : tid, ll, in1);
+        lay[slot][tid] = zsel(in0, n0);
+        if (has1) lay[slot][e1] = zsel(in1, n1);
     };
     // a layer's 3 x 3 neighbourhood enters only through four coefficient-free
     // sums (corners, x and y neighbours, centre), kept instead of the nine values
@@ -390,23 +402,22 @@ __global__ __launch_bounds__(RX * RY) void k_residual3d(int Nx, int Ny, int Nz, 
     const bool out = i < Nx && j < Ny;
     const long id0 = b * N3 + (long)(out ? j : 0) * Nx + (out ? i : 0);
     fetch(l0 - 1);
-    stash(0);
+    stash(0, l0 - 1);
     fetch(l0);
-    stash(1);
+    stash(1, l0);
     fetch(l0 + 1);
-    z2 fn = F[id0 + (long)l0 * Nxy];
+    fn = F[id0 + (long)l0 * Nxy];
     __syncthreads();
     Part pm, pc, pp;
     plane(0, pm);
     plane(1, pc);
+    int sn = 2;   // the slot of layer l+1: that of layer l-2, last read a barrier ago
     for (int l = l0; l < l1; l++) {
-        const int sn = (l - l0 + 2) % 3;   // the slot of layer l-2, last read a barrier ago
-        stash(sn);                         // layer l+1
+        stash(sn, l + 1);
         const z2 f = fn;
-        if (l + 1 < l1) {
-            fetch(l + 2);
-            fn = F[id0 + (long)(l + 1) * Nxy];
-        }
+        // past the chunk's halo: one address, never used
+        fetch(l + 2 <= l1 ? l + 2 : -1);
+        fn = F[id0 + (long)min(l + 1, l1 - 1) * Nxy];
         __syncthreads();
         plane(sn, pp);
         if (out) {
@@ -420,6 +431,7 @@ __global__ __launch_bounds__(RX * RY) void k_residual3d(int Nx, int Ny, int Nz, 
         pc = pp;
         // slot sn is next rewritten two steps on; every thread has passed
         // the next step's barrier, after its read here, by then
+        sn = sn == 2 ? 0 : sn + 1;
     }
 }
 
@@ -444,15 +456,16 @@ hipError_t launch_residual3d(int Nx, int Ny, int Nz, int batch, const void *coef
     const int nchunk = (Nz + RZ - 1) / RZ;
     const int per = 65535 / nchunk;   // right-hand sides per launch (grid z)
     if (per < 1) return hipErrorInvalidValue;
+    const int RX = (Nx + 63) / 64 * 64 > (Nx + 31) / 32 * 32 ? 32 : 64;
     for (int b0 = 0; b0 < batch; b0 += per) {
         const int nb = batch - b0 < per ? batch - b0 : per;
         dim3 g((unsigned)((Nx + RX - 1) / RX), (unsigned)((Ny + RY - 1) / RY), (unsigned)(nchunk * nb));
-        if (res_f32)
-            hipLaunchKernelGGL(k_residual3d<float>, g, dim3(RX, RY), 0, st, Nx, Ny, Nz, nchunk, (const z2 *)coef,
-                               nop, (const z2 *)u, (const z2 *)F, (float2 *)res, b0);
-        else
-            hipLaunchKernelGGL(k_residual3d<double>, g, dim3(RX, RY), 0, st, Nx, Ny, Nz, nchunk, (const z2 *)coef,
-                               nop, (const z2 *)u, (const z2 *)F, (z2 *)res, b0);
+        auto run = [&](auto kfn, auto *out) {
+            hipLaunchKernelGGL(kfn, g, dim3(RX, RY), 0, st, Nx, Ny, Nz, nchunk, (const z2 *)coef, nop, (const z2 *)u,
+                               (const z2 *)F, out, b0);
+        };
+        if (res_f32) run(RX == 64 ? k_residual3d<float, 64> : k_residual3d<float, 32>, (float2 *)res);
+        else run(RX == 64 ? k_residual3d<double, 64> : k_residual3d<double, 32>, (z2 *)res);
     }
     return hipGetLastError();
 }
