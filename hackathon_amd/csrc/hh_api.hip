@@ -1698,29 +1698,30 @@ extern "C" int hh_rhs2d(hh_plan *p, int order, double hx, double hy, const void 
     int rc = set_device(c);
     if (rc) return rc;
     const int Nx = p->Nx, Ny = p->Ny;
-    const long XY = (long)(Nx + 2) * (Ny + 2), wstride = 2 * XY + (long)Nx * Ny;
-    // per-row k^2 and compact (k^2)_y, uploaded after the field work area
-    size_t wbytes = order == 6 ? (size_t)wstride * batch * 16 : 0;
+    // per-row k^2 and compact (k^2)_y
     const int nop = p->nop;
     size_t tbytes = (size_t)2 * Ny * nop * 16;
-    if ((rc = ensure_scratch(c, wbytes + tbytes))) return rc;
+    if ((rc = ensure_scratch(c, tbytes))) return rc;
     // tables [op][j]: k^2 at the interior rows, then compact (k^2)_y
     std::vector<cd> tab(2 * (size_t)Ny * nop);
     std::vector<cd> k2y;
+    int k2y_nonzero = 0;
     for (int o = 0; o < nop; o++) {
         const double *ke = k2e + 2 * (size_t)o * (Ny + 2);
         if (order == 6) k2_y_compact(Ny, hy, ke, k2yb ? k2yb + 4 * (size_t)o : nullptr, k2y);
         for (int j = 0; j < Ny; j++) {
             tab[(size_t)o * Ny + j] = ld(ke, j + 1);
             tab[(size_t)(nop + o) * Ny + j] = order == 6 ? k2y[j] : cd(0);
+            if (order == 6 && k2y[j] != cd(0)) k2y_nonzero = 1;
         }
     }
-    char *tb = (char *)c->scratch + wbytes;
+    char *tb = (char *)c->scratch;
     HIPCHK(hipMemcpyAsync(tb, tab.data(), tbytes, hipMemcpyHostToDevice, c->stream));
     hh::Rhs2D r;
     r.order = order; r.Nx = Nx; r.Ny = Ny; r.batch = batch; r.hx = hx; r.hy = hy;
+    r.k2y_nonzero = k2y_nonzero;
     r.f_e = f_e; r.u_e = u_e; r.fy_b = fy_b; r.fxx_b = fxx_b; r.fyy_b = fyy_b;
-    r.k2c = tb; r.k2y = tb + (size_t)Ny * nop * 16; r.coef = p->coef64; r.nop = nop; r.work = c->scratch;
+    r.k2c = tb; r.k2y = tb + (size_t)Ny * nop * 16; r.coef = p->coef64; r.nop = nop;
     TimeScope ts(c, 4, (double)Nx * Ny * batch * 32);
     hipError_t e = hh::launch_rhs2d(r, F, c->stream);
     if (e != hipSuccess) return fail(HH_ERR_DEVICE, "rhs2d launch failed: %s", hipGetErrorString(e));
@@ -1740,8 +1741,7 @@ extern "C" int hh_rhs3d(hh_plan *p, int order, double hx, double hy, double hz, 
     int rc = set_device(c);
     if (rc) return rc;
     const int Nx = p->Nx, Ny = p->Ny, Nz = p->Nz;
-    const long E = (long)(Nx + 2) * (Ny + 2) * (Nz + 2);
-    size_t wbytes = order == 6 ? (size_t)3 * E * batch * 16 : 0;
+    size_t wbytes = order == 6 ? (size_t)Nx * Ny * Nz * batch * 16 : 0;
     const int nop = p->nop;
     size_t tbytes = (size_t)(2 * Nz + 2) * nop * 16;
     if ((rc = ensure_scratch(c, wbytes + tbytes))) return rc;

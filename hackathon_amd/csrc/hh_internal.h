@@ -113,22 +113,6 @@ struct ModeSet {
 void classify_modes(int dim, int Nx, int Ny, int Nz, int nop, const std::complex<double> *hcoef,
                     const double *lamx, const double *lamy, bool real, double kappa_flag, ModeSet &ms);
 
-// Compact fourth-order derivative line solves (band 1, diag, 1) over an
-// extended-grid field; see CompactProb in hh_tri.hip for the index maps.
-struct Compact {
-    int n, first;
-    double diag, h;
-    const void *f;
-    long field_in, mA, orig, sA, sB, eS;
-    const void *lo, *hi;
-    long field_bnd, bo, bA, bB;
-    void *out;
-    long field_out, oorig, oA, oB, oS;
-    long nmodes;
-    int batch;
-};
-hipError_t launch_compact(const Compact &cd, hipStream_t st);
-
 // Choose a tridiagonal block shape for a system of length n and nmodes modes.
 void tri_shape(int n, long nmodes, int prec, int *W, int *P, int *mmax);
 // LDS bytes of the tridiagonal kernel's reduced system: two buffers of A, C
@@ -151,11 +135,12 @@ struct Rhs2D {
     const void *fyy_b;   // ring
     const void *k2c;     // Ny: k^2 at interior rows
     const void *k2y;     // Ny: compact (k^2)_y at interior rows
+    int k2y_nonzero;     // any of them
     const void *coef;    // Ny x 6 per operator
     int nop;             // right-hand side b uses operator b % nop
-    void *work;          // 2 (Nx+2)(Ny+2)+Nx Ny per rhs
 };
 hipError_t launch_rhs2d(const Rhs2D &r, void *F, hipStream_t st);
+hipError_t launch_rhs2d_6(const Rhs2D &r, void *F, hipStream_t st);   // sixth order (hh_compact.hip)
 
 struct Rhs3D {
     int order, Nx, Ny, Nz, batch;
@@ -166,9 +151,10 @@ struct Rhs3D {
     const void *kz;               // Nz: compact (k^2)_z
     const void *coef;             // Nz x 12 per operator
     int nop;                      // right-hand side b uses operator b % nop
-    void *work;                   // 3 extended fields per rhs
+    void *work;                   // sixth order: one field per rhs
 };
 hipError_t launch_rhs3d(const Rhs3D &r, void *F, hipStream_t st);
+hipError_t launch_rhs3d_6(const Rhs3D &r, void *F, hipStream_t st);   // sixth order (hh_compact.hip)
 
 // res = A u - F (the reference residual.c), and the fused refinement pieces.
 // coef tables: right-hand side b uses coef + (b % nop) * (6 Ny | 12 Nz)

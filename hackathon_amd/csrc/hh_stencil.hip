@@ -4,14 +4,13 @@
 // Right-hand side (kernel set "c"):
 //   2D_Program/main_functions/rhs.c:4-150 with 2D_Program/partial_derivatives
 //   3D_Program/main_functions/rhs.c:13-294 with 3D_Program/partial_derivatives
-// The compact fourth-order derivatives (tridiagonal [1,4,1] and [1,10,1]
-// systems) run on the partitioned tridiagonal kernel (launch_compact); the
-// second-order differences and the final combination are fused into one
-// pointwise pass, which also subtracts the Dirichlet closure.
+// Orders 2 and 4 are pointwise differences, combined with the Dirichlet closure
+// in one pass; the sixth order with its compact derivatives is hh_compact.hip.
 // Residual: 2D_Program/main_functions/residual.c:3-34 (9-point),
 //           3D_Program/main_functions/residual.c:42-96 (27-point).
 #include <type_traits>
 
+#include "hh_closure.h"
 #include "hh_common.h"
 #include "hh_internal.h"
 
@@ -26,34 +25,11 @@ HH_DEV z2 zd(z2 a, z2 b) { return csub<double>(a, b); }
 HH_DEV z2 zm(z2 a, z2 b) { return cmul<double>(a, b); }
 
 // ---------------------------------------------------------------- 2D RHS
-__global__ void k_ring2d(int Nx, int Ny, int batch, const z2 *fxx_b, const z2 *fyy_b, z2 *work, long wstride) {
-    const int X = Nx + 2, Y = Ny + 2;
-    const long XY = (long)X * Y;
-    const int nring = 2 * X + 2 * Y;
-    long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= (long)nring * batch) return;
-    int b = (int)(id / nring), r = (int)(id % nring);
-    z2 *fxx = work + b * wstride, *fyy = fxx + XY;
-    const z2 *rx = fxx_b + (long)b * nring, *ry = fyy_b + (long)b * nring;
-    long o;
-    if (r < X) o = r;                                   // bottom row j = 0
-    else if (r < 2 * X) o = (r - X) + (long)(Y - 1) * X;     // top row j = Ny+1
-    else if (r < 2 * X + Y) o = (long)(r - 2 * X) * X;       // left column i = 0
-    else o = (X - 1) + (long)(r - 2 * X - Y) * X;            // right column i = Nx+1
-    // rows first, then columns (2D_Program/partial_derivatives/
-    // 4th_order_second_derivative.c:41-51); corners coincide analytically
-    if (r < 2 * X && ((r % X) == 0 || (r % X) == X - 1)) return;
-    fxx[o] = rx[r];
-    fyy[o] = ry[r];
-}
-
 struct Rhs2DArgs {
     int order, Nx, Ny;
     double hx, hy;
-    const z2 *f_e, *u_e, *k2c, *k2y, *coef;
+    const z2 *f_e, *u_e, *coef;
     int nop;
-    const z2 *work;
-    long wstride;
 };
 
 __global__ void k_rhs2d_combine(Rhs2DArgs a, long total, z2 *F) {
@@ -66,21 +42,9 @@ __global__ void k_rhs2d_combine(Rhs2DArgs a, long total, z2 *F) {
     const int i = (int)(p % Nx), j = (int)(p / Nx);
     const z2 *f = a.f_e + b * XY;
     const long c0 = (i + 1) + (long)(j + 1) * X;
-    const double hy2 = a.hy * a.hy, hy4 = hy2 * hy2, hx2 = a.hx * a.hx;
+    const double hy2 = a.hy * a.hy;
     z2 v;
-    if (a.order == 6) {                                           // rhs.c:78-86
-        const z2 *fxx = a.work + b * a.wstride, *fyy = fxx + XY, *fy = fyy + XY;
-        z2 fxxxx = zs(za(zd(fxx[c0 - 1], zs(fxx[c0], 2.0)), fxx[c0 + 1]), 1.0 / hx2);
-        z2 fxxyy = zs(za(zd(fxx[c0 - X], zs(fxx[c0], 2.0)), fxx[c0 + X]), 1.0 / hy2);
-        z2 fyyyy = zs(za(zd(fyy[c0 - X], zs(fyy[c0], 2.0)), fyy[c0 + X]), 1.0 / hy2);
-        const long oj = (long)(b % a.nop) * Ny + j;
-        z2 t1 = zm(zd(zr(1.0), zs(a.k2c[oj], hy2 / 20.0)), f[c0]);
-        z2 t2 = zs(za(fxx[c0], fyy[c0]), hy2 / 12.0);
-        z2 t3 = zs(za(fxxxx, fyyyy), hy4 / 360.0);
-        z2 t4 = zs(fxxyy, hy4 / 90.0);
-        z2 t5 = zs(zm(a.k2y[oj], fy[p]), hy4 / 60.0);
-        v = zs(za(za(za(za(t1, t2), t3), t4), t5), hy2);
-    } else if (a.order == 4) {                                    // rhs.c:21-38
+    if (a.order == 4) {                                    // rhs.c:21-38
         z2 s4 = za(za(za(f[c0 - X], f[c0 + X]), f[c0 - 1]), f[c0 + 1]);
         v = zs(za(zs(f[c0], 2.0 / 3.0), zs(s4, 1.0 / 12.0)), hy2);
     } else {                                                      // rhs.c:4-19
@@ -88,104 +52,29 @@ __global__ void k_rhs2d_combine(Rhs2DArgs a, long total, z2 *F) {
     }
     // Dirichlet closure rhs.c:126-148: subtract the stencil weight times u
     // for every neighbour that lies on the boundary
-    if (i == 0 || i == Nx - 1 || j == 0 || j == Ny - 1) {
-        const z2 *u = a.u_e + b * XY;
-        const z2 *cq = a.coef + 6 * ((long)(b % a.nop) * Ny + j);  // bm, am, b, a, bp, ap
-        for (int dj = -1; dj <= 1; dj++)
-            for (int di = -1; di <= 1; di++) {
-                int ii = i + di, jj = j + dj;
-                if (ii >= 0 && ii < Nx && jj >= 0 && jj < Ny) continue;
-                z2 w = dj == 1 ? (di == 0 ? cq[5] : cq[4]) : dj == 0 ? (di == 0 ? cq[3] : cq[2]) : (di == 0 ? cq[1] : cq[0]);
-                v = zd(v, zm(w, u[(ii + 1) + (long)(jj + 1) * X]));
-            }
-    }
+    if (i == 0 || i == Nx - 1 || j == 0 || j == Ny - 1)
+        v = dirichlet2d(v, Nx, Ny, i, j, a.coef + 6 * ((long)(b % a.nop) * Ny + j), a.u_e + b * XY);
     F[id] = v;
 }
 
 hipError_t launch_rhs2d(const Rhs2D &r, void *F, hipStream_t st) {
-    const int Nx = r.Nx, Ny = r.Ny, X = Nx + 2, Y = Ny + 2;
-    const long XY = (long)X * Y, wstride = 2 * XY + (long)Nx * Ny;
-    const int nring = 2 * X + 2 * Y;
-    z2 *work = (z2 *)r.work;
-    hipError_t e;
-    if (r.order == 6) {
-        // fyy: modes i along y, [1,10,1]  (4th_order_second_derivative.c:64-122)
-        Compact c{};
-        c.n = Ny; c.first = 0; c.diag = 10.0; c.h = r.hy;
-        c.f = r.f_e; c.field_in = XY; c.mA = Nx; c.orig = 1; c.sA = 1; c.sB = 0; c.eS = X;
-        c.lo = r.fyy_b; c.hi = (const z2 *)r.fyy_b + X; c.field_bnd = nring; c.bo = 1; c.bA = 1; c.bB = 0;
-        c.out = work + XY; c.field_out = wstride; c.oorig = 1 + X; c.oA = 1; c.oB = 0; c.oS = X;
-        c.nmodes = Nx; c.batch = r.batch;
-        if ((e = launch_compact(c, st)) != hipSuccess) return e;
-        // fy: modes i along y, [1,4,1]  (4th_order_first_derivative.c:36-74)
-        c.first = 1; c.diag = 4.0;
-        c.lo = r.fy_b; c.hi = (const z2 *)r.fy_b + Nx; c.field_bnd = 2 * Nx; c.bo = 0; c.bA = 1; c.bB = 0;
-        c.out = work + 2 * XY; c.oorig = 0; c.oA = 1; c.oB = 0; c.oS = Nx;
-        if ((e = launch_compact(c, st)) != hipSuccess) return e;
-        // fxx: modes j along x, [1,10,1]  (4th_order_second_derivative.c:4-62)
-        Compact d{};
-        d.n = Nx; d.first = 0; d.diag = 10.0; d.h = r.hx;
-        d.f = r.f_e; d.field_in = XY; d.mA = Ny; d.orig = X; d.sA = X; d.sB = 0; d.eS = 1;
-        d.lo = (const z2 *)r.fxx_b + 2 * X; d.hi = (const z2 *)r.fxx_b + 2 * X + Y; d.field_bnd = nring;
-        d.bo = 1; d.bA = 1; d.bB = 0;
-        d.out = work; d.field_out = wstride; d.oorig = X + 1; d.oA = X; d.oB = 0; d.oS = 1;
-        d.nmodes = Ny; d.batch = r.batch;
-        if ((e = launch_compact(d, st)) != hipSuccess) return e;
-        long nr = (long)nring * r.batch;
-        hipLaunchKernelGGL(k_ring2d, dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, st, Nx, Ny, r.batch,
-                           (const z2 *)r.fxx_b, (const z2 *)r.fyy_b, work, wstride);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
+    if (r.order == 6) return launch_rhs2d_6(r, F, st);
+    const int Nx = r.Nx, Ny = r.Ny;
     Rhs2DArgs a;
     a.order = r.order; a.Nx = Nx; a.Ny = Ny; a.hx = r.hx; a.hy = r.hy;
-    a.f_e = (const z2 *)r.f_e; a.u_e = (const z2 *)r.u_e; a.k2c = (const z2 *)r.k2c; a.k2y = (const z2 *)r.k2y;
-    a.coef = (const z2 *)r.coef; a.nop = r.nop > 0 ? r.nop : 1; a.work = work; a.wstride = wstride;
+    a.f_e = (const z2 *)r.f_e; a.u_e = (const z2 *)r.u_e;
+    a.coef = (const z2 *)r.coef; a.nop = r.nop > 0 ? r.nop : 1;
     long total = (long)Nx * Ny * r.batch;
     hipLaunchKernelGGL(k_rhs2d_combine, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, a, total, (z2 *)F);
     return hipGetLastError();
 }
 
 // ---------------------------------------------------------------- 3D RHS
-__global__ void k_fill0(long n, z2 *p) {
-    long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id < n) p[id] = zr(0.0);
-}
-
-// ghost faces of the extended second derivatives: x faces of fxx, y faces
-// of fyy, z faces of fzz (rhs.c:90-109, 4th_order_partials.c:141-146,
-// 208-213, 275-280); all other ghosts stay zero
-__global__ void k_faces3d(int Nx, int Ny, int Nz, int batch, const z2 *fxx_f, const z2 *fyy_f, const z2 *fzz_f,
-                          z2 *work, long wstride) {
-    const long X = Nx + 2, Y = Ny + 2, Z = Nz + 2, XY = X * Y, E = XY * Z;
-    const long nf = 2 * Y * Z + 2 * X * Z + 2 * X * Y;
-    long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= nf * batch) return;
-    int b = (int)(id / nf);
-    long r = id % nf;
-    z2 *w = work + b * wstride;
-    if (r < 2 * Y * Z) {
-        long face = r / (Y * Z), q = r % (Y * Z), j = q % Y, l = q / Y;
-        w[face * (X - 1) + j * X + l * XY] = fxx_f[b * 2 * Y * Z + r];
-        return;
-    }
-    r -= 2 * Y * Z;
-    if (r < 2 * X * Z) {
-        long face = r / (X * Z), q = r % (X * Z), i = q % X, l = q / X;
-        w[E + i + face * (Y - 1) * X + l * XY] = fyy_f[b * 2 * X * Z + r];
-        return;
-    }
-    r -= 2 * X * Z;
-    long face = r / XY, q = r % XY;
-    w[2 * E + q + face * (Z - 1) * XY] = fzz_f[b * 2 * XY + r];
-}
-
 struct Rhs3DArgs {
     int order, Nx, Ny, Nz;
     double hx, hy, hz;
-    const z2 *f_e, *u_e, *k2e, *kz, *coef;
+    const z2 *f_e, *u_e, *coef;
     int nop;
-    const z2 *work;
-    long wstride;
 };
 
 __global__ void k_rhs3d_combine(Rhs3DArgs a, long total, z2 *F) {
@@ -198,85 +87,34 @@ __global__ void k_rhs3d_combine(Rhs3DArgs a, long total, z2 *F) {
     const long i = p % Nx, j = (p / Nx) % Ny, l = p / (Nx * Ny);
     const z2 *f = a.f_e + b * E;
     const long c0 = (i + 1) + (j + 1) * X + (l + 1) * XY;
-    const double hz = a.hz, h2 = hz * hz;
     z2 v;
-    if (a.order == 6) {                                           // rhs.c:150-166
-        const z2 *fxx = a.work + b * a.wstride, *fyy = fxx + E, *fzz = fyy + E;
-        z2 fxxxx = zs(za(zd(fxx[c0 - 1], zs(fxx[c0], 2.0)), fxx[c0 + 1]), 1.0 / (a.hx * a.hx));
-        z2 fyyyy = zs(za(zd(fyy[c0 - X], zs(fyy[c0], 2.0)), fyy[c0 + X]), 1.0 / (a.hy * a.hy));
-        z2 fzzzz = zs(za(zd(fzz[c0 - XY], zs(fzz[c0], 2.0)), fzz[c0 + XY]), 1.0 / h2);
-        z2 fxxyy = zs(za(zd(fxx[c0 - X], zs(fxx[c0], 2.0)), fxx[c0 + X]), 1.0 / (a.hy * a.hy));
-        z2 fxxzz = zs(za(zd(fxx[c0 - XY], zs(fxx[c0], 2.0)), fxx[c0 + XY]), 1.0 / h2);
-        z2 fyyzz = zs(za(zd(fyy[c0 - XY], zs(fyy[c0], 2.0)), fyy[c0 + XY]), 1.0 / h2);
-        const long op = b % a.nop;
-        z2 first = zm(zd(zr(1.0), zs(a.k2e[op * (Nz + 2) + l + 1], h2 / 20.0)), f[c0]);
-        z2 second = zs(za(za(fxx[c0], fyy[c0]), fzz[c0]), h2 / 12.0);
-        z2 third = zs(za(za(fxxxx, fyyyy), fzzzz), h2 * h2 / 360.0);
-        z2 fourth = zs(za(za(fxxyy, fxxzz), fyyzz), h2 * h2 / 90.0);
-        z2 fifth = zs(zm(a.kz[op * Nz + l], zd(f[c0 + XY], f[c0 - XY])), h2 * hz / 120.0);
-        v = za(za(za(za(first, second), third), fourth), fifth);
-    } else if (a.order == 4) {                                    // rhs.c:34-53
+    if (a.order == 4) {                                    // rhs.c:34-53
         z2 s6 = za(za(za(za(za(f[c0 - 1], f[c0 + 1]), f[c0 - X]), f[c0 + X]), f[c0 - XY]), f[c0 + XY]);
         v = za(f[c0], zs(zd(s6, zs(f[c0], 6.0)), 1.0 / 12.0));
     } else {                                                      // rhs.c:13-32
         v = f[c0];
     }
-    // z-face closure (rhs.c:24-29, 55-62, 167-174)
+    // z-face closure (rhs.c:24-29, 55-62)
     if (l == 0 || l == Nz - 1) {
         const z2 *u = a.u_e + b * E;
-        for (int side = 0; side < 2; side++) {
-            if ((side == 0 && l != 0) || (side == 1 && l != Nz - 1)) continue;
-            long g = (i + 1) + (j + 1) * X + (side == 0 ? 0 : (Nz + 1) * XY);
-            if (a.order == 2) {
-                v = zd(v, u[g]);
-            } else {
-                const z2 *cq = a.coef + 12 * ((long)(b % a.nop) * Nz + (side == 0 ? 0 : (Nz - 1))) + (side == 0 ? 8 : 4);
-                z2 corner = za(za(za(u[g - 1 - X], u[g + 1 - X]), u[g - 1 + X]), u[g + 1 + X]);
-                z2 xn = za(u[g - 1], u[g + 1]);
-                z2 yn = za(u[g - X], u[g + X]);
-                z2 w = za(za(za(zm(cq[0], corner), zm(cq[1], xn)), zm(cq[2], yn)), zm(cq[3], u[g]));
-                v = zd(v, w);
-            }
+        const long g = (i + 1) + (j + 1) * X;
+        if (a.order == 2) {
+            if (l == 0) v = zd(v, u[g]);
+            if (l == Nz - 1) v = zd(v, u[g + (Nz + 1) * XY]);
+        } else {
+            v = dirichlet3d(v, X, XY, (int)Nz, (int)l, g, a.coef + 12 * (long)(b % a.nop) * Nz, u);
         }
     }
     F[id] = v;
 }
 
 hipError_t launch_rhs3d(const Rhs3D &r, void *F, hipStream_t st) {
-    const long Nx = r.Nx, Ny = r.Ny, Nz = r.Nz, X = Nx + 2, Y = Ny + 2, Z = Nz + 2, XY = X * Y, E = XY * Z;
-    const long wstride = 3 * E;
-    z2 *work = (z2 *)r.work;
-    hipError_t e;
-    if (r.order == 6) {
-        long nw = wstride * r.batch;
-        hipLaunchKernelGGL(k_fill0, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, st, nw, work);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        long nf = (2 * Y * Z + 2 * X * Z + 2 * X * Y) * r.batch;
-        hipLaunchKernelGGL(k_faces3d, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0, st, r.Nx, r.Ny, r.Nz, r.batch,
-                           (const z2 *)r.fxx_f, (const z2 *)r.fyy_f, (const z2 *)r.fzz_f, work, wstride);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        Compact c{};
-        c.first = 0; c.diag = 10.0; c.f = r.f_e; c.field_in = E; c.field_out = wstride; c.batch = r.batch;
-        // fxx: modes (j, l) along x (4th_order_partials.c:94-160)
-        c.n = r.Nx; c.h = r.hx; c.mA = Ny; c.orig = X + XY; c.sA = X; c.sB = XY; c.eS = 1;
-        c.lo = r.fxx_f; c.hi = (const z2 *)r.fxx_f + Y * Z; c.field_bnd = 2 * Y * Z; c.bo = 1 + Y; c.bA = 1; c.bB = Y;
-        c.out = work; c.oorig = X + XY + 1; c.oA = X; c.oB = XY; c.oS = 1; c.nmodes = Ny * Nz;
-        if ((e = launch_compact(c, st)) != hipSuccess) return e;
-        // fyy: modes (i, l) along y (:162-227)
-        c.n = r.Ny; c.h = r.hy; c.mA = Nx; c.orig = 1 + XY; c.sA = 1; c.sB = XY; c.eS = X;
-        c.lo = r.fyy_f; c.hi = (const z2 *)r.fyy_f + X * Z; c.field_bnd = 2 * X * Z; c.bo = 1 + X; c.bA = 1; c.bB = X;
-        c.out = work + E; c.oorig = 1 + X + XY; c.oA = 1; c.oB = XY; c.oS = X; c.nmodes = Nx * Nz;
-        if ((e = launch_compact(c, st)) != hipSuccess) return e;
-        // fzz: modes (i, j) along z (:229-294)
-        c.n = r.Nz; c.h = r.hz; c.mA = Nx; c.orig = 1 + X; c.sA = 1; c.sB = X; c.eS = XY;
-        c.lo = r.fzz_f; c.hi = (const z2 *)r.fzz_f + XY; c.field_bnd = 2 * XY; c.bo = 1 + X; c.bA = 1; c.bB = X;
-        c.out = work + 2 * E; c.oorig = 1 + X + XY; c.oA = 1; c.oB = X; c.oS = XY; c.nmodes = Nx * Ny;
-        if ((e = launch_compact(c, st)) != hipSuccess) return e;
-    }
+    if (r.order == 6) return launch_rhs3d_6(r, F, st);
+    const long Nx = r.Nx, Ny = r.Ny, Nz = r.Nz;
     Rhs3DArgs a;
     a.order = r.order; a.Nx = r.Nx; a.Ny = r.Ny; a.Nz = r.Nz; a.hx = r.hx; a.hy = r.hy; a.hz = r.hz;
-    a.f_e = (const z2 *)r.f_e; a.u_e = (const z2 *)r.u_e; a.k2e = (const z2 *)r.k2e; a.kz = (const z2 *)r.kz;
-    a.coef = (const z2 *)r.coef; a.nop = r.nop > 0 ? r.nop : 1; a.work = work; a.wstride = wstride;
+    a.f_e = (const z2 *)r.f_e; a.u_e = (const z2 *)r.u_e;
+    a.coef = (const z2 *)r.coef; a.nop = r.nop > 0 ? r.nop : 1;
     long total = Nx * Ny * Nz * r.batch;
     hipLaunchKernelGGL(k_rhs3d_combine, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, a, total, (z2 *)F);
     return hipGetLastError();

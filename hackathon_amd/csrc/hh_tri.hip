@@ -193,57 +193,6 @@ template <typename T, typename Ti, typename To, int DIM, bool REAL> struct HelmP
     }
 };
 
-// Compact fourth-order derivative of a field sampled on the extended grid
-// (2D_Program/partial_derivatives/4th_order_*.c, 3D_Program/
-// partial_derivatives/4th_order_partials.c:94-294): band (1, diag, 1),
-//   second derivative (diag 10): rhs = 12 (f_{q+1} - 2 f_q + f_{q-1}) / h^2
-//   first derivative  (diag 4):  rhs = 3 (f_{q+1} - f_{q-1}) / h
-// minus the analytic boundary value at q = 0 and q = n-1.  Mode m maps to
-// the extended-grid line origin + (m % mA) sA + (m / mA) sB; element q sits
-// at (q+1) eS along it.  The result goes to oorig + (m%mA) oA + (m/mA) oB + q oS.
-template <typename T> struct CompactProb {
-    using OT = T;   // bands (1, diag, 1)
-    int nn, first;
-    T diag, h;
-    const C2<T> *f;
-    long field_in, field_out, field_bnd;
-    long mA, orig, sA, sB, eS;
-    const C2<T> *lo, *hi;   // boundary values, indexed bo + (m%mA) bA + (m/mA) bB
-    long bo, bA, bB;
-    C2<T> *out;
-    long oorig, oA, oB, oS;
-    struct Mode { long in, bnd, out; };
-    HH_DEV int n() const { return nn; }
-    HH_DEV Mode mode(long m, int) const {
-        long a = m % mA, b = m / mA;
-        Mode md;
-        md.in = orig + a * sA + b * sB;
-        md.bnd = bo + a * bA + b * bB;
-        md.out = oorig + a * oA + b * oB;
-        return md;
-    }
-    HH_DEV Band<T> band(const Mode &, int q) const {
-        Band<T> r;
-        r.sub = q > 0 ? (T)1 : (T)0;
-        r.dia = diag;
-        r.sup = q < nn - 1 ? (T)1 : (T)0;
-        return r;
-    }
-    HH_DEV C2<T> rhs(int bt, const Mode &md, int q) const {
-        const C2<T> *g = f + bt * field_in + md.in + (long)(q + 1) * eS;
-        C2<T> v;
-        if (first) v = cscale<T>(csub<T>(g[eS], g[-eS]), (T)3 / h);
-        else v = cscale<T>(cadd<T>(csub<T>(g[eS], cscale<T>(g[0], (T)2)), g[-eS]), (T)12 / (h * h));
-        if (q == 0) v = csub<T>(v, lo[bt * field_bnd + md.bnd]);
-        if (q == nn - 1) v = csub<T>(v, hi[bt * field_bnd + md.bnd]);
-        return v;
-    }
-    HH_DEV void store(int bt, const Mode &md, int q, C2<T> x) const {
-        out[bt * field_out + md.out + (long)q * oS] = x;
-    }
-    HH_DEV bool skip(int, long) const { return false; }
-};
-
 // Blocks are dealt round-robin to the 8 XCDs (block b runs on XCD b % 8).
 // Neighbouring mode tiles share cache lines when W*sizeof(complex) < 128,
 // so tiles are renumbered to run consecutively on one XCD and its L2.
@@ -908,31 +857,6 @@ hipError_t launch_tri_seq(const TriHelm &t, DstTypes ty, const void *in, void *o
     if (ty.in == 0 && ty.out == 0) return launch_seq_t<double, double>(t, in, out, st);
     if (ty.in == 1 && ty.out == 1) return launch_seq_t<float, float>(t, in, out, st);
     return hipErrorInvalidValue;
-}
-
-hipError_t launch_compact(const Compact &cd, hipStream_t st) {
-    CompactProb<double> pb;
-    pb.nn = cd.n;
-    pb.first = cd.first;
-    pb.diag = cd.diag;
-    pb.h = cd.h;
-    pb.f = (const double2 *)cd.f;
-    pb.field_in = cd.field_in;
-    pb.field_out = cd.field_out;
-    pb.field_bnd = cd.field_bnd;
-    pb.mA = cd.mA; pb.orig = cd.orig; pb.sA = cd.sA; pb.sB = cd.sB; pb.eS = cd.eS;
-    pb.lo = (const double2 *)cd.lo; pb.hi = (const double2 *)cd.hi;
-    pb.bo = cd.bo; pb.bA = cd.bA; pb.bB = cd.bB;
-    pb.out = (double2 *)cd.out;
-    pb.oorig = cd.oorig; pb.oA = cd.oA; pb.oB = cd.oB; pb.oS = cd.oS;
-    int W, P, mm;
-    tri_shape(cd.n, cd.nmodes, F64, &W, &P, &mm);
-    switch (mm) {
-    case 4: return launch_tri_nr<double, 4, 1>(pb, cd.n, cd.nmodes, cd.batch, 1, W, P, st);
-    case 8: return launch_tri_nr<double, 8, 1>(pb, cd.n, cd.nmodes, cd.batch, 1, W, P, st);
-    case 16: return launch_tri_nr<double, 16, 1>(pb, cd.n, cd.nmodes, cd.batch, 1, W, P, st);
-    default: return hipErrorInvalidValue;
-    }
 }
 
 hipError_t launch_tri_helm(const TriHelm &t, DstTypes ty, const void *in, void *out, hipStream_t st) {
