@@ -1057,16 +1057,6 @@ extern "C" int hh_plan_set_tile_width(hh_plan *p, int tw) {
     return HH_OK;
 }
 
-// Built-in shape of FP64 elimination on FP32 storage (mixed precision), on
-// top of the FP64 one: in 3D from n = 255, 16 rows per thread (255^3: W = 16,
-// 114 against 137 us per launch for 8 rows).
-static void fp32_storage_rows(const hh_plan *p, int n, long nmodes, hh::TriHelm &t) {
-    if (p->dim == 3 && t.mmax == 8 && n >= 255) {
-        t.mmax = 16;
-        hh::tri_shape_rows(n, nmodes, 16, &t.W, &t.P);
-    }
-}
-
 // Shape of `rows` rows per thread and about `threads` threads per block:
 // W the largest power of two with W P <= threads, in [wmin, 16], and no
 // more than the modes need.
@@ -1082,9 +1072,8 @@ static void shape_for(int n, long nmodes, int rows, int threads, int wmin, hh::T
 }
 
 // Built-in block shape of the mode solves (W, P, rows and right-hand sides
-// per thread).  kind 0: FP64 elimination on FP64 storage, 1: FP64
-// elimination on FP32 storage, 2: FP32 elimination; per_op: right-hand
-// sides per operator in the batch.  Measured on MI355X (order-6 operators
+// per thread) for FP64 or FP32 elimination; per_op: right-hand sides per
+// operator in the batch.  Measured on MI355X (order-6 operators
 // with k^2 = 2500 or 2500 + 50i, row-major spectrum; microseconds of the
 // mode pass of one solve, near-resonant modes included; in brackets the
 // former rule of 256-thread blocks, 16 rows per thread above n = 512):
@@ -1104,33 +1093,21 @@ static void shape_for(int n, long nmodes, int rows, int threads, int wmin, hh::T
 //         449 (506), 2047 x 16: 609 (733), 511: 131 (133), 255: 51 (53)
 // and the former rule elsewhere (within 2% of the best shape measured).
 // Two right-hand sides per thread need two per operator in the batch.
-static void builtin_tri_shape(const hh_plan *p, int kind, long per_op, bool real, hh::TriHelm &t) {
+static void builtin_tri_shape(const hh_plan *p, bool f32, long per_op, bool real, hh::TriHelm &t) {
     const int n = p->dim == 2 ? p->Ny : p->Nz;
     const long nmodes = p->dim == 2 ? p->Nx : (long)p->Nx * p->Ny;
-    hh::tri_shape(n, nmodes, kind == 0 ? hh::F64 : hh::F32, &t.W, &t.P, &t.mmax);
+    hh::tri_shape(n, nmodes, &t.W, &t.P, &t.mmax);
     t.nr = 1;
-    if (kind == 1) {
-        hh::tri_shape(n, nmodes, hh::F64, &t.W, &t.P, &t.mmax);
-        fp32_storage_rows(p, n, nmodes, t);
-        // real bands, 16 rows: two right-hand sides per thread share the
-        // operator's pivots (N=1023 x 64: 419 against 531 us per launch)
-        // when the grid still has 8 blocks per CU or more
-        if (real && t.mmax == 16 && per_op >= 2) {
-            const long tiles = (nmodes + t.W - 1) / t.W;
-            if (tiles * p->nop * ((per_op + 1) / 2) >= 2048) t.nr = 2;
-        }
-        return;
-    }
     if (n <= 16) return;
     int nr = 1;
-    if (kind == 0 && real && p->dim == 2) {
+    if (!f32 && real && p->dim == 2) {
         if (n <= 512) { shape_for(n, nmodes, 16, 512, 1, t); nr = 2; }
         else if (n <= 1024) shape_for(n, nmodes, 8, 512, 1, t);
         else { shape_for(n, nmodes, 16, 512, 1, t); nr = 2; }
-    } else if (kind == 0 && real) {
+    } else if (!f32 && real) {
         if (n <= 128) { shape_for(n, nmodes, 8, 128, 1, t); nr = 2; }
         else { shape_for(n, nmodes, 16, 256, 1, t); nr = 2; }
-    } else if (kind == 0) {
+    } else if (!f32) {
         if (n <= 512) { shape_for(n, nmodes, 8, 256, 1, t); nr = 2; }
         else shape_for(n, nmodes, 16, 256, 4, t);
     } else if (real && p->dim == 2) {
@@ -1146,7 +1123,7 @@ extern "C" int hh_plan_get_tri_shape(const hh_plan *p, int *W, int *P, int *rows
     int n = p->dim == 2 ? p->Ny : p->Nz;
     // the shape of the solve's elimination (mixed precision: FP32), for a
     // batch of two or more right-hand sides per operator
-    builtin_tri_shape(p, p->prec == HH_PREC_MIXED ? 2 : 0, 2, p->real_op && p->real_mode != 0, t);
+    builtin_tri_shape(p, p->prec == HH_PREC_MIXED, 2, p->real_op && p->real_mode != 0, t);
     if (p->tri_W > 0) {   // the tuned shape, where its reduced system fits the LDS (as in solve_core)
         const bool mixed = p->prec == HH_PREC_MIXED, real = p->real_op && p->real_mode != 0;
         const int nr = mixed ? 1 : p->tri_nr;
@@ -1223,11 +1200,12 @@ static int solve_core(hh_plan *p, int ti, int tc, int to, int tri_comp, const vo
     t.real = p->real_op && p->real_mode != 0;
     t.coefr = tri_comp == 0 ? p->coefr64 : p->coefr32;
     t.nop = p->nop;
+    t.uni = p->d_bits;
     t.cstride = p->dim == 2 ? 6L * Ny : 12L * Nz;
     t.lamx = p->lamx; t.lamy = p->lamy;
     int n = p->dim == 2 ? Ny : Nz;
     const long per_op = (batch + p->nop - 1) / p->nop;
-    builtin_tri_shape(p, tri_comp == 1 ? 2 : tc == 1 ? 1 : 0, per_op, t.real, t);
+    builtin_tri_shape(p, tri_comp == 1, per_op, t.real, t);
     if (p->tri_W > 0 && p->tri_mm > 0) {   // shape chosen by the autotuner
         const int nr = tri_comp == 0 ? p->tri_nr : 1;
         int P = (n + p->tri_mm - 1) / p->tri_mm;
@@ -1244,7 +1222,7 @@ static int solve_core(hh_plan *p, int ti, int tc, int to, int tri_comp, const vo
     // factors (FP64 arithmetic), then the partitioned kernel for the rest
     t.nfx = p->ms.nfx;
     if (t.nfx > 0) {
-        t.fbits = p->d_bits;
+        t.fbits = p->d_bits + p->nop;
         t.fwords = p->ms.words;
         t.foff = p->d_foff;
         t.fmode = p->d_fmode;

@@ -76,6 +76,7 @@ struct TriHelm {
     int tiled = 0;      // field in the mode-tiled layout of the row DSTs: tile width (a multiple of W), 0 = row-major
     int real = 0;       // every coefficient real: use coefr, the real parts in pairs ([q][3] / [q][6] complex slots)
     const void *coefr = nullptr;
+    const uint32_t *uni = nullptr;  // per operator: every row of its table is the same (device)
     // Near-resonant modes (ModeSet below): the partitioned kernel does not
     // store them (bit m % 32 of fbits[o * fwords + m / 32] set); they are
     // solved by the sequential kernel from the factors in fac.
@@ -103,7 +104,7 @@ struct ModeSet {
     int n = 0, nop = 0, words = 0, nfx = 0;
     long nmodes = 0;
     std::vector<int> foff, fmode;         // per operator offsets (nop + 1), flagged modes
-    std::vector<uint32_t> bits;           // [op][words]
+    std::vector<uint32_t> bits;           // [op] every row of its table is the same, then [op][words] flagged modes
     std::vector<std::complex<double>> facc;   // [entry][row](L, P, R, Up)
     std::vector<double> facr;             // real parts (real operators only)
     std::vector<int> singular;            // per operator
@@ -114,7 +115,7 @@ void classify_modes(int dim, int Nx, int Ny, int Nz, int nop, const std::complex
                     const double *lamx, const double *lamy, bool real, double kappa_flag, ModeSet &ms);
 
 // Choose a tridiagonal block shape for a system of length n and nmodes modes.
-void tri_shape(int n, long nmodes, int prec, int *W, int *P, int *mmax);
+void tri_shape(int n, long nmodes, int *W, int *P, int *mmax);
 // LDS bytes of the tridiagonal kernel's reduced system: two buffers of A, C
 // (operator values of op bytes) and nr complex right-hand sides (cx bytes).
 inline size_t tri_lds_bytes(size_t op, size_t cx, int P, int W, int nr) {

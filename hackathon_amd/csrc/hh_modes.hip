@@ -191,7 +191,7 @@ void classify_modes(int dim, int Nx, int Ny, int Nz, int nop, const cd *hcoef, c
     ms.words = (int)((nmodes + 31) / 32);
     ms.foff.assign(nop + 1, 0);
     ms.fmode.clear();
-    ms.bits.assign((size_t)nop * ms.words, 0u);
+    ms.bits.assign((size_t)nop * (1 + ms.words), 0u);
     ms.facc.clear();
     ms.facr.clear();
     ms.singular.assign(nop, 0);
@@ -206,6 +206,7 @@ void classify_modes(int dim, int Nx, int Ny, int Nz, int nop, const cd *hcoef, c
         for (int q = 1; q < n && uniform; q++)
             for (int t = 0; t < nc; t++)
                 if (tab[(long)q * nc + t] != tab[t]) { uniform = false; break; }
+        ms.bits[o] = uniform;
         ms.foff[o] = (int)ms.fmode.size();
         for (long m = 0; m < nmodes; m++) {
             const double lx = dim == 2 ? lamx[m] : lamx[m % Nx];
@@ -248,7 +249,7 @@ void classify_modes(int dim, int Nx, int Ny, int Nz, int nop, const cd *hcoef, c
             if (!flag) continue;
             const long e = (long)ms.fmode.size();
             ms.fmode.push_back((int)m);
-            ms.bits[(size_t)o * ms.words + m / 32] |= 1u << (m % 32);
+            ms.bits[nop + (size_t)o * ms.words + m / 32] |= 1u << (m % 32);
             ms.facc.resize((size_t)(e + 1) * n * 4);
             cd *fc = ms.facc.data() + (size_t)e * n * 4;
             bool ok;

@@ -60,20 +60,26 @@ template <typename T> struct OpAr<T, C2<T>> {
     }
     static HH_DEV O fms2(O a, O b, O d, O e, O c) { return csub<T>(c, cadd<T>(cmul<T>(a, b), cmul<T>(d, e))); }
 };
+// Real: the fused operations are written out and nothing else is contracted, so
+// that both forms of the bands (one per mode, one per row) round alike.
+HH_DEV double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+HH_DEV float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+#pragma clang fp contract(off)
 template <typename T> struct OpAr<T, T> {
     using O = T;
     static HH_DEV O zero() { return (T)0; }
     static HH_DEV O one() { return (T)1; }
     static HH_DEV O mul(O a, O b) { return a * b; }
     static HH_DEV O neg(O a) { return -a; }
-    static HH_DEV O fms(O a, O b, O c) { return c - a * b; }
+    static HH_DEV O fms(O a, O b, O c) { return fma_(-a, b, c); }
     // rcp_nr's Newton steps hold for either sign of a nonzero argument
     static HH_DEV O rcp(O a) { return rcp_nr(a); }
     static HH_DEV C2<T> xmul(O a, C2<T> x) { return mk<T>(a * x.x, a * x.y); }
-    static HH_DEV C2<T> xfms(O a, C2<T> x, C2<T> y) { return mk<T>(y.x - a * x.x, y.y - a * x.y); }
+    static HH_DEV C2<T> xfms(O a, C2<T> x, C2<T> y) { return mk<T>(fma_(-a, x.x, y.x), fma_(-a, x.y, y.y)); }
     static HH_DEV C2<T> xfms2(O a, C2<T> x, O b, C2<T> z, C2<T> y) { return xfms(b, z, xfms(a, x, y)); }
     static HH_DEV O fms2(O a, O b, O d, O e, O c) { return fms(d, e, fms(a, b, c)); }
 };
+#pragma clang fp contract(fast)
 
 template <typename T, int DIM, bool REAL> struct HelmBands {
     using OT = typename std::conditional<REAL, T, C2<T>>::type;
@@ -99,47 +105,57 @@ template <typename T, int DIM, bool REAL> struct HelmBands {
     // Bands in the reference's operation order with no fused multiply-adds
     // (2D_Program/main_functions/LU.c:16-23, 3D_Program/main_functions/
     // LU.c:34-47): the FP64 bands equal the reference's to the last bit.
-    HH_DEV Band<OT> band(const Mode &md, int q) const {
+    // raw: from table row q, as if it had both neighbours.
+    HH_DEV Band<OT> raw(const Mode &md, int q) const {
 #pragma clang fp contract(off)
         Band<OT> r;
-        const T ms = q > 0 ? (T)1 : (T)0, ps = q < n - 1 ? (T)1 : (T)0;
         if constexpr (REAL) {
             if constexpr (DIM == 2) {   // pairs (bm, am), (b, a), (bp, ap)
                 const C2<T> *c = md.cf + 3 * (long)q;
                 const T l = md.l0;
                 const C2<T> c0 = c[0], c1 = c[1], c2 = c[2];
-                r.sub = ms * (c0.x * l + c0.y);
+                r.sub = c0.x * l + c0.y;
                 r.dia = c1.x * l + c1.y;
-                r.sup = ps * (c2.x * l + c2.y);
+                r.sup = c2.x * l + c2.y;
             } else {   // pairs (a, b), (c, d), (ap, bp), (cp, dp), (am, bm), (cm, dm)
                 const C2<T> *c = md.cf + 6 * (long)q;
                 const T a = md.l0, b = md.l1, g = md.l2;
                 const C2<T> c0 = c[0], c1 = c[1], c2 = c[2], c3 = c[3], c4 = c[4], c5 = c[5];
                 r.dia = c0.x * a + c0.y * b + c1.x * g + c1.y;
-                r.sup = ps * (c2.x * a + c2.y * b + c3.x * g + c3.y);
-                r.sub = ms * (c4.x * a + c4.y * b + c5.x * g + c5.y);
+                r.sup = c2.x * a + c2.y * b + c3.x * g + c3.y;
+                r.sub = c4.x * a + c4.y * b + c5.x * g + c5.y;
             }
         } else if constexpr (DIM == 2) {
             const C2<T> *c = md.cf + 6 * (long)q;
             const T l = md.l0;
-            r.sub = mk<T>(ms * (c[0].x * l + c[1].x), ms * (c[0].y * l + c[1].y));
+            r.sub = mk<T>(c[0].x * l + c[1].x, c[0].y * l + c[1].y);
             r.dia = mk<T>(c[2].x * l + c[3].x, c[2].y * l + c[3].y);
-            r.sup = mk<T>(ps * (c[4].x * l + c[5].x), ps * (c[4].y * l + c[5].y));
+            r.sup = mk<T>(c[4].x * l + c[5].x, c[4].y * l + c[5].y);
         } else {
             const C2<T> *c = md.cf + 12 * (long)q;
             const T a = md.l0, b = md.l1, g = md.l2;
             r.dia = mk<T>(c[0].x * a + c[1].x * b + c[2].x * g + c[3].x, c[0].y * a + c[1].y * b + c[2].y * g + c[3].y);
-            r.sup = mk<T>(ps * (c[4].x * a + c[5].x * b + c[6].x * g + c[7].x),
-                          ps * (c[4].y * a + c[5].y * b + c[6].y * g + c[7].y));
-            r.sub = mk<T>(ms * (c[8].x * a + c[9].x * b + c[10].x * g + c[11].x),
-                          ms * (c[8].y * a + c[9].y * b + c[10].y * g + c[11].y));
+            r.sup = mk<T>(c[4].x * a + c[5].x * b + c[6].x * g + c[7].x, c[4].y * a + c[5].y * b + c[6].y * g + c[7].y);
+            r.sub = mk<T>(c[8].x * a + c[9].x * b + c[10].x * g + c[11].x,
+                          c[8].y * a + c[9].y * b + c[10].y * g + c[11].y);
+        }
+        return r;
+    }
+    // the first row has no sub-, the last no superdiagonal
+    HH_DEV Band<OT> ends(Band<OT> r, int q) const {
+        const T ms = q > 0 ? (T)1 : (T)0, ps = q < n - 1 ? (T)1 : (T)0;
+        if constexpr (REAL) {
+            r.sub *= ms;
+            r.sup *= ps;
+        } else {
+            r.sub = cscale<T>(r.sub, ms);
+            r.sup = cscale<T>(r.sup, ps);
         }
         return r;
     }
 };
 
 // Helmholtz problem: bands from HelmBands, right-hand side and solution in
-// the row-major field (element (b, m, q) at b*field + m + q*S).
 // the row-major field (element (b, m, q) at b*field + m + q*S), or, with
 // tw > 0, the mode-tiled one the row DSTs write for it (tiles of tw
 // neighbouring modes, tile t0 = m & ~(tw-1) holding its modes for all n rows
@@ -154,6 +170,7 @@ template <typename T, typename Ti, typename To, int DIM, bool REAL> struct HelmP
     int tw;
     const uint32_t *fbits;   // near-resonant modes, solved by k_tri_seq: not stored here
     int fwords;
+    const uint32_t *uni;     // per operator: every row of its table is the same
     struct Mode { typename HelmBands<T, DIM, REAL>::Mode bm; long off, step; };
     HH_DEV int n() const { return bands.n; }
     HH_DEV Mode mode(long m, int bt) const {
@@ -169,7 +186,9 @@ template <typename T, typename Ti, typename To, int DIM, bool REAL> struct HelmP
         }
         return md;
     }
-    HH_DEV Band<OT> band(const Mode &md, int q) const { return bands.band(md.bm, q); }
+    HH_DEV Band<OT> raw(const Mode &md, int q) const { return bands.raw(md.bm, q); }
+    HH_DEV Band<OT> ends(Band<OT> r, int q) const { return bands.ends(r, q); }
+    HH_DEV bool uniform(int o) const { return uni[o] != 0; }
     HH_DEV C2<T> rhs(int b, const Mode &md, int q) const {
         return cconv<T, Ti>(in[b * field + md.off + (long)q * md.step]);
     }
@@ -209,8 +228,8 @@ HH_DEV long xcd_tile(long b, long G) {
 // recurrences are repeated.  Block (mode tile, y): operator o = y % nop,
 // right-hand sides o + nop (NR (y / nop) + r), r < NR, those past the batch
 // are computed on a clamped index and not stored.
-template <typename T, int MMAX, int NR, int NT, class Prob>
-__global__ __launch_bounds__(NT) void k_tri(Prob prob, long nmodes, int W, int P, int batch, int nop, int g0) {
+template <typename T, int MMAX, int NR, bool UNI, class Prob>
+HH_DEV void tri_block(const Prob &prob, long nmodes, int W, int P, int batch, int nop, int g0) {
     using OT = typename Prob::OT;
     using O = OpAr<T, OT>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -257,7 +276,15 @@ __global__ __launch_bounds__(NT) void k_tri(Prob prob, long nmodes, int W, int P
     for (int r = 0; r < NR; r++)
 #pragma unroll
         for (int t = 0; t < MMAX; t++) db[r][t] = prob.rhs(bidx[r], md, min(s + t, e));
-    const Band<OT> bs = prob.band(md, s);
+    // An operator whose table rows are all equal (constant k) has one band per
+    // mode: its 3 (2D) or 6 (3D) loads are made once, not per row.
+    Band<OT> same;
+    if constexpr (UNI) same = prob.raw(md, 0);
+    auto band = [&](int q) {
+        if constexpr (UNI) return prob.ends(same, q);
+        else return prob.ends(prob.raw(md, q), q);
+    };
+    const Band<OT> bs = band(s);
     const OT sub_s = bs.sub, dia_s = bs.dia, sup_s = bs.sup;
     C2<T> d_s[NR];
 #pragma unroll
@@ -271,7 +298,7 @@ __global__ __launch_bounds__(NT) void k_tri(Prob prob, long nmodes, int W, int P
     for (int r = 0; r < NR; r++) pd[r] = mk<T>(0, 0);
 #pragma unroll
     for (int t = 1; t < MMAX; t++) {
-        const Band<OT> bq = prob.band(md, min(s + t, e));
+        const Band<OT> bq = band(min(s + t, e));
         const OT a = bq.sub;
         const OT den = (t == 1) ? bq.dia : O::fms(a, pc, bq.dia);
         const OT rc = O::rcp(den);
@@ -424,6 +451,22 @@ __global__ __launch_bounds__(NT) void k_tri(Prob prob, long nmodes, int W, int P
         }
         prob.store(b, md, e, xe);
     }
+}
+
+// Real operators whose table rows are all equal (constant k) take one band per
+// mode, others one per row; which, is read from the device beside the tables,
+// so that recorded work follows operators replaced later.  Both forms give the
+// same bits.  Loads per row were what the pass waited for: 64 x 1023^2 599 ->
+// 551 us, 2047^2 x 6 308 -> 263, 255^3 156 -> 103 (5.1 TB/s), 125^3 24.0 -> 19.2.
+template <typename T, int MMAX, int NR, int NT, class Prob>
+__global__ __launch_bounds__(NT) void k_tri(Prob prob, long nmodes, int W, int P, int batch, int nop, int g0) {
+    if constexpr (std::is_same<typename Prob::OT, T>::value) {
+        if (prob.uniform(blockIdx.y % nop)) {
+            tri_block<T, MMAX, NR, true>(prob, nmodes, W, P, batch, nop, g0);
+            return;
+        }
+    }
+    tri_block<T, MMAX, NR, false>(prob, nmodes, W, P, batch, nop, g0);
 }
 
 // Near-resonant modes: the reference's substitution (2D_Program/
@@ -693,7 +736,7 @@ static hipError_t launch_tri_prob(const Prob &pb, int n, long nmodes, int batch,
     return hipErrorInvalidValue;
 }
 
-void tri_shape(int n, long nmodes, int prec, int *W, int *P, int *mmax) {
+void tri_shape(int n, long nmodes, int *W, int *P, int *mmax) {
     // Measured on MI355X (FP64, k = 50 compact operators, row-major field):
     // 256-thread blocks win at every length tried; 16 rows per thread above
     // n = 512 (fewer chunks, a shallower reduced system), 8 below.  n = 1023,
@@ -702,7 +745,6 @@ void tri_shape(int n, long nmodes, int prec, int *W, int *P, int *mmax) {
     // 207 us against 283 us for 16 x 8.
     int mm = n > 512 ? 16 : 8;
     if (n <= 16) mm = 4;
-    (void)prec;
     tri_shape_rows(n, nmodes, mm, W, P);
     *mmax = mm;
 }
@@ -751,6 +793,7 @@ static hipError_t launch_tri_r(const TriHelm &t, const void *in, void *out, hipS
     pb.tw = t.tiled;
     pb.fbits = t.fbits;
     pb.fwords = t.fwords;
+    pb.uni = t.uni;
     if (t.tiled && ((t.tiled & (t.tiled - 1)) || t.tiled % t.W)) return hipErrorInvalidValue;
     return launch_tri_prob<T, MM>(pb, pb.bands.n, nmodes, t.batch, pb.bands.nop, t.W, t.P, t.nr, st);
 }
@@ -789,6 +832,7 @@ static hipError_t launch_seq_rc(const TriHelm &t, const void *in, void *out, hip
     pb.tw = t.tiled;
     pb.fbits = nullptr;
     pb.fwords = 0;
+    pb.uni = nullptr;
     const int n = pb.bands.n;
     constexpr int PW = 64 / C;
     const int G = ((n + R - 1) / R + PW - 1) / PW * PW;   // positions, whole waves
@@ -862,7 +906,6 @@ hipError_t launch_tri_seq(const TriHelm &t, DstTypes ty, const void *in, void *o
 hipError_t launch_tri_helm(const TriHelm &t, DstTypes ty, const void *in, void *out, hipStream_t st) {
     if (ty.comp == 0 && ty.in == 0 && ty.out == 0) return launch_tri_mm<double, double, double>(t, in, out, st);
     if (ty.comp == 1 && ty.in == 1 && ty.out == 1) return launch_tri_mm<float, float, float>(t, in, out, st);
-    if (ty.comp == 0 && ty.in == 1 && ty.out == 1) return launch_tri_mm<double, float, float>(t, in, out, st);
     return hipErrorInvalidValue;
 }
 
