@@ -150,12 +150,13 @@ struct hh_plan {
     // factors (hh_modes.hip), with their device copies
     double kappa_flag = hh::HH_KAPPA_FLAG;
     hh::ModeSet ms;
-    int *d_foff = nullptr, *d_fmode = nullptr;
+    int2 *d_ent = nullptr;                       // [op][nfx] (mode, entry)
+    std::vector<int2> hent;
     uint32_t *d_bits = nullptr;
     void *d_facc = nullptr, *d_facr = nullptr;
     std::vector<cd> hfacc_t;                     // staging of the device layout
     std::vector<double> hfacr_t;
-    size_t cap_foff = 0, cap_fmode = 0, cap_bits = 0, cap_facc = 0, cap_facr = 0;
+    size_t cap_ent = 0, cap_bits = 0, cap_facc = 0, cap_facr = 0;
     // Generation: bumped whenever a change would invalidate a recorded graph
     // (device tables reallocated, band kind, operator count or launch shapes
     // changed); graphs record it at capture and refuse to replay a newer plan.
@@ -785,8 +786,11 @@ static int upload_modes(hh_plan *p) {
                 p->hfacc_t[(q * ne + e) * 4 + k] = m.facc[(e * n + q) * 4 + k];
                 if (!m.facr.empty()) p->hfacr_t[(q * ne + e) * 4 + k] = m.facr[(e * n + q) * 4 + k];
             }
-    if ((rc = ensure_dev(p, (void **)&p->d_foff, &p->cap_foff, m.foff.size() * sizeof(int)))) return rc;
-    if ((rc = ensure_dev(p, (void **)&p->d_fmode, &p->cap_fmode, m.fmode.size() * sizeof(int)))) return rc;
+    // one row of nfx entries per operator, padded with (-1, 0)
+    p->hent.assign((size_t)m.nop * m.nfx, make_int2(-1, 0));
+    for (int o = 0; o < m.nop; o++)
+        for (int e = m.foff[o]; e < m.foff[o + 1]; e++) p->hent[(size_t)o * m.nfx + e - m.foff[o]] = make_int2(m.fmode[e], e);
+    if ((rc = ensure_dev(p, (void **)&p->d_ent, &p->cap_ent, p->hent.size() * sizeof(int2)))) return rc;
     if ((rc = ensure_dev(p, (void **)&p->d_bits, &p->cap_bits, m.bits.size() * sizeof(uint32_t)))) return rc;
     if ((rc = ensure_dev(p, &p->d_facc, &p->cap_facc, m.facc.size() * sizeof(cd)))) return rc;
     if ((rc = ensure_dev(p, &p->d_facr, &p->cap_facr, m.facr.size() * sizeof(double)))) return rc;
@@ -794,8 +798,7 @@ static int upload_modes(hh_plan *p) {
         if (bytes) HIPCHK(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, c->stream));
         return HH_OK;
     };
-    if ((rc = cp(p->d_foff, m.foff.data(), m.foff.size() * sizeof(int)))) return rc;
-    if ((rc = cp(p->d_fmode, m.fmode.data(), m.fmode.size() * sizeof(int)))) return rc;
+    if ((rc = cp(p->d_ent, p->hent.data(), p->hent.size() * sizeof(int2)))) return rc;
     if ((rc = cp(p->d_bits, m.bits.data(), m.bits.size() * sizeof(uint32_t)))) return rc;
     if ((rc = cp(p->d_facc, p->hfacc_t.data(), p->hfacc_t.size() * sizeof(cd)))) return rc;
     return cp(p->d_facr, p->hfacr_t.data(), p->hfacr_t.size() * sizeof(double));
@@ -974,8 +977,7 @@ extern "C" int hh_plan_destroy(hh_plan *p) {
     dev_free(c, p->coefr32, (size_t)nc * n * p->cap_nop * 4);
     dev_free(c, p->lamx, (size_t)p->Nx * 8);
     if (p->lamy) dev_free(c, p->lamy, (size_t)p->Ny * 8);
-    dev_free(c, p->d_foff, p->cap_foff);
-    dev_free(c, p->d_fmode, p->cap_fmode);
+    dev_free(c, p->d_ent, p->cap_ent);
     dev_free(c, p->d_bits, p->cap_bits);
     dev_free(c, p->d_facc, p->cap_facc);
     dev_free(c, p->d_facr, p->cap_facr);
@@ -1219,25 +1221,18 @@ static int solve_core(hh_plan *p, int ti, int tc, int to, int tri_comp, const vo
         }
     }
     // near-resonant modes: reference-order substitution from the host's
-    // factors (FP64 arithmetic), then the partitioned kernel for the rest
+    // factors (FP64 arithmetic), beside the partitioned elimination of the rest
     t.nfx = p->ms.nfx;
     if (t.nfx > 0) {
         t.fbits = p->d_bits + p->nop;
         t.fwords = p->ms.words;
-        t.foff = p->d_foff;
-        t.fmode = p->d_fmode;
+        t.ent = p->d_ent;
         t.fac = t.real ? p->d_facr : p->d_facc;
         t.nent = (long)p->ms.fmode.size();
     }
-    // The two kernels touch disjoint outputs (the partitioned kernel reads the
-    // near-resonant modes' rows but does not store them).  Run concurrently on
-    // a second stream they took as long together (C2: 651 us) as one after
-    // the other: the partitioned kernel's blocks fill the chip.
     auto tri = [&](void *buf) -> int {
         TimeScope ts(c, 2, (double)t.field * batch * (tc ? 16 : 32));
-        hipError_t e = hh::launch_tri_seq(t, hh::DstTypes{tc, 0, tc}, buf, buf, c->stream);
-        if (e != hipSuccess) return fail(HH_ERR_DEVICE, "near-resonant mode launch failed: %s", hipGetErrorString(e));
-        e = hh::launch_tri_helm(t, hh::DstTypes{tc, tri_comp, tc}, buf, buf, c->stream);
+        hipError_t e = hh::launch_tri_helm(t, hh::DstTypes{tc, tri_comp, tc}, buf, buf, c->stream);
         if (e != hipSuccess) return fail(HH_ERR_DEVICE, "tridiagonal launch failed: %s", hipGetErrorString(e));
         return HH_OK;
     };

@@ -79,20 +79,15 @@ struct TriHelm {
     const uint32_t *uni = nullptr;  // per operator: every row of its table is the same (device)
     // Near-resonant modes (ModeSet below): the partitioned kernel does not
     // store them (bit m % 32 of fbits[o * fwords + m / 32] set); they are
-    // solved by the sequential kernel from the factors in fac.
+    // solved in the reference's order, beside it, from the factors in fac.
     const uint32_t *fbits = nullptr;
     int fwords = 0;
-    const int *foff = nullptr, *fmode = nullptr;   // per operator: entries foff[o] .. foff[o+1]-1, their modes
-    const void *fac = nullptr;                     // [row][entry](L, P, R, Up): double (real) or double2
+    const int2 *ent = nullptr;                     // [op][nfx] (mode, index of its factors), (-1, 0) past the operator's last
+    const void *fac = nullptr;                     // [row][index](L, P, R, Up): double (real) or double2
     int nfx = 0;                                   // most entries of one operator
     long nent = 0;                                 // entries of all operators
 };
 hipError_t launch_tri_helm(const TriHelm &t, DstTypes ty, const void *in, void *out, hipStream_t st);
-// Sequential reference-order substitution of the near-resonant modes of t
-// (FP64 arithmetic; storage as ty.in / ty.out); run before launch_tri_helm
-// on the same buffer.  No-op when t.nfx == 0.
-hipError_t launch_tri_seq(const TriHelm &t, DstTypes ty, const void *in, void *out, hipStream_t st);
-
 // A mode whose condition estimate exceeds this is singular to working
 // precision (no correct digit is left in FP64).
 constexpr double HH_SINGULAR_KAPPA = 1e14;

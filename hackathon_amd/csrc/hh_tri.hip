@@ -161,29 +161,38 @@ template <typename T, int DIM, bool REAL> struct HelmBands {
 // neighbouring modes, tile t0 = m & ~(tw-1) holding its modes for all n rows
 // contiguously: b*field + t0*n + q*w + (m - t0), w = min(tw, nmodes - t0)),
 // where each thread's rows are whole w*16-byte segments one after another.
-template <typename T, typename Ti, typename To, int DIM, bool REAL> struct HelmProb {
+template <typename T_, typename Ti_, typename To_, int DIM_, bool REAL_> struct HelmProb {
+    using T = T_;
+    using Ti = Ti_;
+    using To = To_;
+    static constexpr int DIM = DIM_;
+    static constexpr bool REAL = REAL_;
     using OT = typename HelmBands<T, DIM, REAL>::OT;
     HelmBands<T, DIM, REAL> bands;
     const C2<Ti> *in;
     C2<To> *out;
     long field, S, nmodes;
     int tw;
-    const uint32_t *fbits;   // near-resonant modes, solved by k_tri_seq: not stored here
+    const uint32_t *fbits;   // near-resonant modes, solved by chain_block: not stored by tri_block
     int fwords;
     const uint32_t *uni;     // per operator: every row of its table is the same
     struct Mode { typename HelmBands<T, DIM, REAL>::Mode bm; long off, step; };
     HH_DEV int n() const { return bands.n; }
+    // where mode m's rows lie in a field
+    HH_DEV void place(long m, long &off, long &step) const {
+        if (tw == 0) {
+            off = m;
+            step = S;
+        } else {
+            const long t0 = m & ~(long)(tw - 1);
+            step = min((long)tw, nmodes - t0);
+            off = t0 * bands.n + (m - t0);
+        }
+    }
     HH_DEV Mode mode(long m, int bt) const {
         Mode md;
         md.bm = bands.mode(m, bt);
-        if (tw == 0) {
-            md.off = m;
-            md.step = S;
-        } else {
-            const long t0 = m & ~(long)(tw - 1);
-            md.step = min((long)tw, nmodes - t0);
-            md.off = t0 * bands.n + (m - t0);
-        }
+        place(m, md.off, md.step);
         return md;
     }
     HH_DEV Band<OT> raw(const Mode &md, int q) const { return bands.raw(md.bm, q); }
@@ -196,20 +205,6 @@ template <typename T, typename Ti, typename To, int DIM, bool REAL> struct HelmP
         out[b * field + md.off + (long)q * md.step] = cconv<To, T>(x);
     }
     HH_DEV bool skip(int o, long m) const { return fbits && ((fbits[(long)o * fwords + (m >> 5)] >> (m & 31)) & 1u); }
-    // FP64 access of the sequential kernel
-    HH_DEV double2 rhs64(int b, const Mode &md, int q) const {
-        return cconv<double, Ti>(in[b * field + md.off + (long)q * md.step]);
-    }
-    HH_DEV void store64(int b, const Mode &md, int q, double2 x) const {
-        out[b * field + md.off + (long)q * md.step] = cconv<To, double>(x);
-    }
-    // one part (comp 0 real, 1 imaginary) of an element, as FP64
-    HH_DEV double rhs64c(int b, const Mode &md, int q, int comp) const {
-        return (double)reinterpret_cast<const Ti *>(in + b * field + md.off + (long)q * md.step)[comp];
-    }
-    HH_DEV void store64c(int b, const Mode &md, int q, int comp, double v) const {
-        reinterpret_cast<To *>(out + b * field + md.off + (long)q * md.step)[comp] = (To)v;
-    }
 };
 
 // Blocks are dealt round-robin to the 8 XCDs (block b runs on XCD b % 8).
@@ -229,7 +224,7 @@ HH_DEV long xcd_tile(long b, long G) {
 // right-hand sides o + nop (NR (y / nop) + r), r < NR, those past the batch
 // are computed on a clamped index and not stored.
 template <typename T, int MMAX, int NR, bool UNI, class Prob>
-HH_DEV void tri_block(const Prob &prob, long nmodes, int W, int P, int batch, int nop, int g0) {
+HH_DEV void tri_block(const Prob &prob, long nmodes, int W, int P, int batch, int nop, int g0, int by, int gy) {
     using OT = typename Prob::OT;
     using O = OpAr<T, OT>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -249,8 +244,8 @@ HH_DEV void tri_block(const Prob &prob, long nmodes, int W, int P, int batch, in
     // before this pass wrote the last right-hand sides last, so they are the
     // ones still in the memory-side cache when the pass starts (and the
     // first ones this pass writes last, where the next row transform starts)
-    const int ng = (int)(gridDim.y / nop);
-    const int o = blockIdx.y % nop, jg = g0 + (ng - 1 - (int)(blockIdx.y / nop));
+    const int ng = gy / nop;
+    const int o = by % nop, jg = g0 + (ng - 1 - by / nop);
     int bidx[NR];
     bool bok[NR];
 #pragma unroll
@@ -266,6 +261,7 @@ HH_DEV void tri_block(const Prob &prob, long nmodes, int W, int P, int batch, in
     const int s = (int)(((long)cq * n) / P), e = (int)(((long)(cq + 1) * n) / P) - 1;
     const int len = e - s + 1;   // 2 <= len <= MMAX
     const auto md = prob.mode(m < nmodes ? m : nmodes - 1, bidx[0]);
+    const bool skip = prob.skip(o, m < nmodes ? m : nmodes - 1);   // asked for early: the stores wait for it
 
     // 0. issue every right-hand-side load of the chunk up front (rows past
     //    e repeat row e), so that the HBM latency is paid once per chunk and
@@ -434,7 +430,7 @@ HH_DEV void tri_block(const Prob &prob, long nmodes, int W, int P, int batch, in
     }
 #pragma unroll
     for (int r = 0; r < NR; r++) { D0[r] = PD[0][r]; D1[r] = PD[1][r]; }
-    if (!valid || prob.skip(o, m)) return;
+    if (!valid || skip) return;
     // 4. back-substitution of the interior and store
 #pragma unroll
     for (int r = 0; r < NR; r++) {
@@ -453,22 +449,6 @@ HH_DEV void tri_block(const Prob &prob, long nmodes, int W, int P, int batch, in
     }
 }
 
-// Real operators whose table rows are all equal (constant k) take one band per
-// mode, others one per row; which, is read from the device beside the tables,
-// so that recorded work follows operators replaced later.  Both forms give the
-// same bits.  Loads per row were what the pass waited for: 64 x 1023^2 599 ->
-// 551 us, 2047^2 x 6 308 -> 263, 255^3 156 -> 103 (5.1 TB/s), 125^3 24.0 -> 19.2.
-template <typename T, int MMAX, int NR, int NT, class Prob>
-__global__ __launch_bounds__(NT) void k_tri(Prob prob, long nmodes, int W, int P, int batch, int nop, int g0) {
-    if constexpr (std::is_same<typename Prob::OT, T>::value) {
-        if (prob.uniform(blockIdx.y % nop)) {
-            tri_block<T, MMAX, NR, true>(prob, nmodes, W, P, batch, nop, g0);
-            return;
-        }
-    }
-    tri_block<T, MMAX, NR, false>(prob, nmodes, W, P, batch, nop, g0);
-}
-
 // Near-resonant modes: the reference's substitution (2D_Program/
 // solver_functions/solver.c:71-86, 3D_Program/solver_functions/
 // solver.c:356-369) in its own operation order, with the factors the host
@@ -482,33 +462,29 @@ __global__ __launch_bounds__(NT) void k_tri(Prob prob, long nmodes, int W, int P
 // q0 = a r, q = q0 + (a - p q0) r with r = RN(1/p) from the host and the
 // residual exact by a fused multiply-add (Markstein).
 //
-// The recurrences are sequential, so the parallelism is across chains (one
-// chain = one near-resonant mode of one right-hand side): a block runs C
-// chains side by side, lane l holding chain l % C and, at position l / C
-// of its wave, R consecutive rows in registers (all loads issued up
-// front).  The chains' positions are walked in order: the C lanes of one
-// position run their rows while the others wait, then hand the carried
-// value to the next position by a lane shuffle, and from wave to wave
-// through LDS.  Block x runs items x C .. x C + C - 1, item = b nfx + e_o,
-// right-hand side b, its operator's near-resonant entry e_o.
-template <typename OT> struct SeqOps;
-template <> struct SeqOps<double> {   // real factors, complex right-hand sides
-    static HH_DEV double zero() { return 0.0; }
-    static HH_DEV double one() { return 1.0; }
-    static HH_DEV double2 fms(double a, double2 x, double2 y) {   // y - a x
+// The recurrences are sequential, so the parallelism is across chains.  A chain
+// is one near-resonant mode of one right-hand side, or, with real factors, one
+// part of it: the real and imaginary parts follow independent recurrences, and
+// apart they have half the instructions per row on the walk's critical path.
+template <typename OT, typename V> struct SeqOps;
+template <> struct SeqOps<double, double> {   // real factors, one part of the right-hand side
+    static HH_DEV double fms(double a, double x, double y) {   // y - a x
 #pragma clang fp contract(off)
-        return mk<double>(y.x - a * x.x, y.y - a * x.y);
+        return y - a * x;
     }
-    static HH_DEV double2 mul(double a, double2 x) { return mk<double>(a * x.x, a * x.y); }
-    static HH_DEV double q1(double a, double p, double r) {
+    static HH_DEV double mul(double a, double x) { return a * x; }
+    static HH_DEV double div(double a, double p, double r) {
         const double q0 = a * r;
         return __builtin_fma(__builtin_fma(-p, q0, a), r, q0);
     }
-    static HH_DEV double2 div(double2 a, double p, double r) { return mk<double>(q1(a.x, p, r), q1(a.y, p, r)); }
 };
-template <> struct SeqOps<double2> {   // complex factors: C99 products, quotients through the reciprocal
-    static HH_DEV double2 zero() { return mk<double>(0, 0); }
-    static HH_DEV double2 one() { return mk<double>(1, 0); }
+template <> struct SeqOps<double, double2> {   // both parts
+    using P = SeqOps<double, double>;
+    static HH_DEV double2 fms(double a, double2 x, double2 y) { return mk<double>(P::fms(a, x.x, y.x), P::fms(a, x.y, y.y)); }
+    static HH_DEV double2 mul(double a, double2 x) { return mk<double>(a * x.x, a * x.y); }
+    static HH_DEV double2 div(double2 a, double p, double r) { return mk<double>(P::div(a.x, p, r), P::div(a.y, p, r)); }
+};
+template <> struct SeqOps<double2, double2> {   // complex factors: C99 products, quotients through the reciprocal
     static HH_DEV double2 mul(double2 a, double2 x) {
 #pragma clang fp contract(off)
         return mk<double>(a.x * x.x - a.y * x.y, a.x * x.y + a.y * x.x);
@@ -520,48 +496,89 @@ template <> struct SeqOps<double2> {   // complex factors: C99 products, quotien
     }
     static HH_DEV double2 div(double2 a, double2, double2 r) { return mul(r, a); }
 };
+HH_DEV double real_of(double v, double) { return v; }
+HH_DEV double2 real_of(double v, double2) { return mk<double>(v, 0); }   // a real as either type
+// a or b by value (a conditional between named vectors selects an address and puts them in scratch)
+HH_DEV double pick(bool c, double a, double b) { return c ? a : b; }
+HH_DEV double2 pick(bool c, double2 a, double2 b) { return mk<double>(c ? a.x : b.x, c ? a.y : b.y); }
+HH_DEV double shift(double v, int k, bool up) { return up ? __shfl_up(v, k, 64) : __shfl_down(v, k, 64); }
+HH_DEV double2 shift(double2 v, int k, bool up) { return mk<double>(shift(v.x, k, up), shift(v.y, k, up)); }
 
-HH_DEV double2 shfl_up2(double2 v, int k) { return mk<double>(__shfl_up(v.x, k, 64), __shfl_up(v.y, k, 64)); }
-HH_DEV double2 shfl_down2(double2 v, int k) { return mk<double>(__shfl_down(v.x, k, 64), __shfl_down(v.y, k, 64)); }
+// The chains of a launch: `blocks` blocks of C chains each (a power of two),
+// in the first `rows` grid rows.  Chain = parts (b nfx + x) + part (parts: 2 where the real and imaginary part
+// are chains of their own, else 1): right-hand side b, its operator's near-resonant entry x, at ent[o nfx + x] = (mode, factors'
+// index) or (-1, 0) where the operator has fewer.
+struct Chains {
+    const int2 *ent;
+    const void *fac;   // [row][index](L, P, R, Up)
+    long nent, blocks;
+    int nfx, C, rows;
+};
 
-template <int R, int C, bool DIV, class Prob, typename OT>
-__global__ __launch_bounds__(512) void k_tri_seq(Prob prob, const int *foff, const int *fmode, const OT *fac,
-                                                 long nent, int nfx, int batch, int nop) {
-    using S = SeqOps<OT>;
-    constexpr int PW = 64 / C;   // positions per wave
-    __shared__ double2 carry[C];
-    const int n = prob.n();
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, NW = blockDim.x >> 6;
-    const int c = lane % C, pw = lane / C;
+// One block of chains.  Lane l holds chain l % C and, at position l / C of its
+// wave, R consecutive rows in registers (all loads issued up front).  A chain's
+// positions are walked in order: the C lanes of one position run their rows
+// while the others wait, then hand the carried value to the next position by a
+// lane shuffle, and from wave to wave through LDS.
+template <int R, bool SPLIT, class Prob>
+HH_DEV void chain_block(const Prob &prob, const Chains &ch, long block, int batch, int nop) {
+    using OT = typename std::conditional<Prob::REAL, double, double2>::type;
+    using V = typename std::conditional<SPLIT, double, double2>::type;
+    using S = SeqOps<OT, V>;
+    constexpr int parts = SPLIT ? 2 : 1;
+    const V zero = real_of(0.0, V());
+    const OT fzero = real_of(0.0, OT()), fone = real_of(1.0, OT());
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    V *carry = reinterpret_cast<V *>(smem_raw);   // C values
+    const int n = prob.n(), C = ch.C, PW = 64 / C;   // positions per wave
+    const int NW = ((n + R - 1) / R + PW - 1) / PW;   // waves with rows
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    if (wave >= NW && NW == 1) return;   // one wave walks alone, without barriers
+    const int c = lane & (C - 1), pw = lane / C;
     const int s = (wave * PW + pw) * R;   // first row of this lane
-    const long item = (long)blockIdx.x * C + c;
-    const int b = (int)(item / nfx), x = (int)(item % nfx);
-    const int o = b < batch ? b % nop : 0;
-    const bool live = b < batch && x < foff[o + 1] - foff[o];
-    // idle chains of the last block run on a valid item and store nothing
-    const int bb = live ? b : 0, e = live ? foff[o] + x : 0;
-    const auto md = prob.mode(fmode[e], bb);
+    const long chain = block * C + c, item = chain / parts;
+    const int part = (int)(chain % parts);
+    int b, x;
+    if (item <= 0x7fffffff) {   // as 32-bit division: a chain's latency counts
+        b = (int)((unsigned)item / (unsigned)ch.nfx);
+        x = (int)((unsigned)item - (unsigned)b * (unsigned)ch.nfx);
+    } else {
+        b = (int)(item / ch.nfx);
+        x = (int)(item % ch.nfx);
+    }
+    // idle chains of the last block and of shorter operators run on a valid entry and store nothing
+    const bool in = b < batch;
+    const int bb = in ? b : 0;
+    const int2 en = ch.ent[(long)(bb % nop) * ch.nfx + (in ? x : 0)];
+    const bool live = in && en.x >= 0;
+    long off, step;
+    prob.place(live ? en.x : 0, off, step);
+    off += bb * prob.field;
+    const OT *fac = reinterpret_cast<const OT *>(ch.fac) + (long)en.y * 4;
     // Rows past n (the tail of the last position) become identity rows
     // (d = 0, L = 0, P = R = 1, Up = 0): the forward walk ends on them with a
     // carry nobody reads, the backward walk leaves them with 0, as it starts,
     // so every real row keeps its bits, and the walks need no per-row branch.
-    double2 d[R];
+    V d[R];
     OT L[R], Pv[R], Rv[R], Up[R];
 #pragma unroll
     for (int i = 0; i < R; i++) {
         const int q = min(s + i, n - 1);
         const bool pad = s + i >= n;
-        const double2 v = prob.rhs64(bb, md, q);
-        const OT *f = fac + ((long)q * nent + e) * 4;
+        const auto *src = prob.in + off + q * step;
+        V v;
+        if constexpr (SPLIT) v = (double)reinterpret_cast<const typename Prob::Ti *>(src)[part];
+        else v = mk<double>((double)src->x, (double)src->y);
+        const OT *f = fac + (long)q * ch.nent * 4;
         const OT f0 = f[0], f1 = f[1], f2 = f[2], f3 = f[3];
-        d[i] = pad ? mk<double>(0, 0) : v;
-        L[i] = pad ? S::zero() : f0;
-        Pv[i] = pad ? S::one() : f1;
-        Rv[i] = pad ? S::one() : f2;
-        Up[i] = pad ? S::zero() : f3;
+        d[i] = pick(pad, zero, v);
+        L[i] = pick(pad, fzero, f0);
+        Pv[i] = pick(pad, fone, f1);
+        Rv[i] = pick(pad, fone, f2);
+        Up[i] = pick(pad, fzero, f3);
     }
     // forward: y_q = d_q - L_q y_{q-1} (L_0 = 0)
-    double2 cy = mk<double>(0, 0);
+    V cy = zero;
     for (int w = 0; w < NW; w++) {
         if (wave == w) {
             if (w > 0) cy = carry[c];
@@ -574,13 +591,13 @@ __global__ __launch_bounds__(512) void k_tri_seq(Prob prob, const int *foff, con
                     }
                     if (pp == PW - 1) carry[c] = cy;
                 }
-                if (pp < PW - 1) cy = shfl_up2(cy, C);
+                if (pp < PW - 1) cy = shift(cy, C, true);
             }
         }
-        __syncthreads();
+        if (NW > 1) __syncthreads();
     }
     // backward: x_q = (y_q - Up_q x_{q+1}) / U_q (2D) or * U_q (3D) (Up_{n-1} = 0)
-    cy = mk<double>(0, 0);
+    cy = zero;
     for (int w = NW - 1; w >= 0; w--) {
         if (wave == w) {
             if (w < NW - 1) cy = carry[c];
@@ -588,119 +605,144 @@ __global__ __launch_bounds__(512) void k_tri_seq(Prob prob, const int *foff, con
                 if (pw == pp) {
 #pragma unroll
                     for (int i = R - 1; i >= 0; i--) {
-                        const double2 a = S::fms(Up[i], cy, d[i]);
-                        if constexpr (DIV) d[i] = S::div(a, Pv[i], Rv[i]);
+                        const V a = S::fms(Up[i], cy, d[i]);
+                        if constexpr (Prob::DIM == 2) d[i] = S::div(a, Pv[i], Rv[i]);
                         else d[i] = S::mul(Rv[i], a);
                         cy = d[i];
                     }
                     if (pp == 0) carry[c] = cy;
                 }
-                if (pp > 0) cy = shfl_down2(cy, C);
+                if (pp > 0) cy = shift(cy, C, false);
             }
         }
-        __syncthreads();
+        if (NW > 1) __syncthreads();
     }
     if (!live) return;
-#pragma unroll
-    for (int i = 0; i < R; i++)
-        if (s + i < n) prob.store64(b, md, s + i, d[i]);
-}
-
-// Real factors: the real and imaginary parts of a right-hand side follow
-// two independent real recurrences with the same factors, so neighbouring
-// lanes run them as separate chains (chain = 2 item + part): half the
-// instructions per row on the walk's critical path, each operation the one
-// k_tri_seq applies to that part (same bits).
-HH_DEV double fms1(double a, double x, double y) {   // y - a x, unfused
-#pragma clang fp contract(off)
-    return y - a * x;
-}
-
-template <int R, int C, bool DIV, class Prob>
-__global__ __launch_bounds__(512) void k_tri_seq_re(Prob prob, const int *foff, const int *fmode, const double *fac,
-                                                    long nent, int nfx, int batch, int nop) {
-    constexpr int PW = 64 / C;   // positions per wave
-    __shared__ double carry[C];
-    const int n = prob.n();
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, NW = blockDim.x >> 6;
-    const int c = lane % C, pw = lane / C;
-    const int s = (wave * PW + pw) * R;   // first row of this lane
-    const long chain = (long)blockIdx.x * C + c;
-    const long item = chain >> 1;
-    const int comp = (int)(chain & 1);
-    const int b = (int)(item / nfx), x = (int)(item % nfx);
-    const int o = b < batch ? b % nop : 0;
-    const bool live = b < batch && x < foff[o + 1] - foff[o];
-    const int bb = live ? b : 0, e = live ? foff[o] + x : 0;
-    const auto md = prob.mode(fmode[e], bb);
-    // rows past n: identity rows, as in k_tri_seq
-    double d[R], L[R], Pv[R], Rv[R], Up[R];
 #pragma unroll
     for (int i = 0; i < R; i++) {
-        const int q = min(s + i, n - 1);
-        const bool pad = s + i >= n;
-        const double v = prob.rhs64c(bb, md, q, comp);
-        const double *f = fac + ((long)q * nent + e) * 4;
-        const double f0 = f[0], f1 = f[1], f2 = f[2], f3 = f[3];
-        d[i] = pad ? 0.0 : v;
-        L[i] = pad ? 0.0 : f0;
-        Pv[i] = pad ? 1.0 : f1;
-        Rv[i] = pad ? 1.0 : f2;
-        Up[i] = pad ? 0.0 : f3;
+        if (s + i >= n) break;
+        auto *dst = prob.out + off + (s + i) * step;
+        using To = typename Prob::To;
+        if constexpr (SPLIT) reinterpret_cast<To *>(dst)[part] = (To)d[i];
+        else *dst = mk<To>((To)d[i].x, (To)d[i].y);
     }
-    double cy = 0.0;
-    for (int w = 0; w < NW; w++) {
-        if (wave == w) {
-            if (w > 0) cy = carry[c];
-            for (int pp = 0; pp < PW; pp++) {
-                if (pw == pp) {
-#pragma unroll
-                    for (int i = 0; i < R; i++) {
-                        d[i] = fms1(L[i], cy, d[i]);
-                        cy = d[i];
-                    }
-                    if (pp == PW - 1) carry[c] = cy;
-                }
-                if (pp < PW - 1) cy = __shfl_up(cy, C, 64);
-            }
+}
+
+// Many chains: a launch of their own, both parts of a value in a lane and as
+// many neighbouring modes side by side as 512 threads hold (whole cache lines a
+// row).  64 x 1023^2, 1152 modes: 60 us before the elimination's 551; beside it
+// as half as wide blocks of split chains the two took 618.
+template <int R, class Prob>
+__global__ __launch_bounds__(512) void k_chains(Prob prob, int batch, int nop, Chains ch) {
+    chain_block<R, false>(prob, ch, blockIdx.x, batch, nop);
+}
+
+// Rows per lane of a chain: as many as a thread of the elimination holds, 8
+// where that would set the kernel's registers (complex factors, FP32 storage).
+template <typename T, int MMAX, class Prob> constexpr int chain_rows() {
+    return MMAX > 8 && !(Prob::REAL && sizeof(T) == 8) ? 8 : MMAX;
+}
+
+// The mode solves of a right-hand-side slice.  The first grid rows hold the
+// near-resonant modes' chains (up to one block per CU), the others the
+// partitioned elimination of the rest: the two touch disjoint outputs (tri_block
+// reads the near-resonant rows, which chain_block rewrites, but does not store
+// what it makes of them), so the chains' latency runs beside the elimination
+// instead of before it: one right-hand side at n = 100: 8.3 + 7.4 -> 7.2 us;
+// 6 x 1023^2: 37 + 53 -> 59; 6 x 2047^2: 64 + 263 -> 273; complex, 12 x 511 x 640:
+// 50 + 74 -> 89.
+//
+// Real operators whose table rows are all equal (constant k) take one band per
+// mode, others one per row; which, is read from the device beside the tables,
+// so that recorded work follows operators replaced later.  Both forms give the
+// same bits.  Loads per row were what the pass waited for: 64 x 1023^2 599 ->
+// 551 us, 2047^2 x 6 308 -> 263, 255^3 156 -> 103 to 125 (4.2 to 5.1 TB/s), 125^3
+// 24.0 -> 19.2.
+template <typename T, int MMAX, int NR, int NT, class Prob>
+__global__ __launch_bounds__(NT) void k_tri(Prob prob, long nmodes, int W, int P, int batch, int nop, int g0, Chains ch) {
+    const int by = (int)blockIdx.y - ch.rows, gy = (int)gridDim.y - ch.rows;
+    if (by < 0) {
+        const long id = (long)blockIdx.y * gridDim.x + blockIdx.x;
+        if (id < ch.blocks) chain_block<chain_rows<T, MMAX, Prob>(), Prob::REAL>(prob, ch, id, batch, nop);
+        return;
+    }
+    if constexpr (Prob::REAL) {
+        if (prob.uniform(by % nop)) {
+            tri_block<T, MMAX, NR, true>(prob, nmodes, W, P, batch, nop, g0, by, gy);
+            return;
         }
-        __syncthreads();
     }
-    cy = 0.0;
-    for (int w = NW - 1; w >= 0; w--) {
-        if (wave == w) {
-            if (w < NW - 1) cy = carry[c];
-            for (int pp = PW - 1; pp >= 0; pp--) {
-                if (pw == pp) {
-#pragma unroll
-                    for (int i = R - 1; i >= 0; i--) {
-                        const double a = fms1(Up[i], cy, d[i]);
-                        if constexpr (DIV) d[i] = SeqOps<double>::q1(a, Pv[i], Rv[i]);
-                        else d[i] = Rv[i] * a;
-                        cy = d[i];
-                    }
-                    if (pp == 0) carry[c] = cy;
-                }
-                if (pp > 0) cy = __shfl_down(cy, C, 64);
-            }
-        }
-        __syncthreads();
-    }
-    if (!live) return;
-#pragma unroll
-    for (int i = 0; i < R; i++)
-        if (s + i < n) prob.store64c(b, md, s + i, comp, d[i]);
+    tri_block<T, MMAX, NR, false>(prob, nmodes, W, P, batch, nop, g0, by, gy);
+}
+
+// Most chains, a power of two up to 64, whose g positions each fit a block of `threads` threads.
+static int chains_in(int g, int threads) {
+    int C = 64;
+    while (C > 1 && (g + 64 / C - 1) / (64 / C) * 64 > threads) C /= 2;
+    return C;
+}
+
+// 16 rows per lane with real factors; 8 with complex ones (twice the
+// registers), except above n = 4096 where 512 threads need 16
+template <int R, class Prob> static hipError_t launch_chains(const Prob &pb, Chains ch, long items, int batch, hipStream_t st) {
+    const int g = (pb.bands.n + R - 1) / R;
+    ch.C = chains_in(g, 512);
+    ch.blocks = (items + ch.C - 1) / ch.C;
+    if (ch.blocks > 0x7fffffffL) return hipErrorInvalidValue;
+    const int threads = (g + 64 / ch.C - 1) / (64 / ch.C) * 64;
+    if (threads > 512) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_chains<R, Prob>), dim3((unsigned)ch.blocks), dim3(threads), 64 * sizeof(double2), st, pb, batch,
+                       pb.bands.nop, ch);
+    return hipGetLastError();
 }
 
 template <typename T, int MM, int NR, class Prob>
-static hipError_t launch_tri_nr(const Prob &pb, int n, long nmodes, int batch, int nop, int W, int P,
-                                hipStream_t st) {
+static hipError_t launch_tri_nr(const Prob &pb, const TriHelm &t, hipStream_t st) {
+    const int n = pb.bands.n, W = t.W, P = t.P, batch = t.batch, nop = pb.bands.nop;
+    const long nmodes = pb.nmodes;
     if (n < 2 || batch < 1 || nop < 1) return hipErrorInvalidValue;
     // every chunk needs at least two rows, at most MM rows
     if (P < 1 || P > n / 2 || (n + P - 1) / P > MM || W * P > 1024) return hipErrorInvalidValue;
     int threads = ((W * P + 63) / 64) * 64;
-    const size_t shm = tri_lds_bytes(sizeof(typename Prob::OT), sizeof(C2<T>), P, W, NR);
+    size_t shm = tri_lds_bytes(sizeof(typename Prob::OT), sizeof(C2<T>), P, W, NR);
     if (shm > 160 * 1024) return hipErrorInvalidValue;
+    if (nop > 65535) return hipErrorInvalidValue;
+    const int per_op = (batch + nop - 1) / nop;
+    const int groups = (per_op + NR - 1) / NR;
+    // grid y holds at most 65535 blocks: launch the right-hand-side groups in
+    // slices, the last slice first (the kernel walks its groups backwards too)
+    const int gmax = 65535 / nop;
+    const int g_first = ((groups - 1) / gmax) * gmax;
+    const unsigned gx = (unsigned)((nmodes + W - 1) / W);
+    Chains ch{};
+    if (t.nfx > 0) {
+        if (!t.ent || !t.fac) return hipErrorInvalidValue;
+        ch.ent = t.ent;
+        ch.fac = t.fac;
+        ch.nent = t.nent;
+        ch.nfx = t.nfx;
+        const long items = (long)t.nfx * batch;
+        // Beside the elimination where one block per CU holds the chains: alone
+        // in a wave (no barrier in the walk) if the blocks suffice, else as many
+        // as the block's waves hold.  More take a launch of their own.
+        constexpr int R = chain_rows<T, MM, Prob>();
+        const int g = (n + R - 1) / R;   // positions of one chain
+        const int wide = threads < g ? (g + 63) / 64 * 64 : threads;
+        const long chains = items * (Prob::REAL ? 2 : 1);
+        ch.C = chains_in(g, 64);
+        if (g > 64 || (chains + ch.C - 1) / ch.C > 256) ch.C = chains_in(g, wide);
+        ch.blocks = (chains + ch.C - 1) / ch.C;
+        if (ch.blocks <= 256 && wide <= 1024 && nop * (groups - g_first) + (ch.blocks + gx - 1) / gx <= 65535) {
+            ch.rows = (int)((ch.blocks + gx - 1) / gx);
+            threads = wide;
+            if (shm < 64 * sizeof(double2)) shm = 64 * sizeof(double2);
+        } else {
+            hipError_t e;
+            if constexpr (Prob::REAL) e = launch_chains<16>(pb, ch, items, batch, st);
+            else e = n > 4096 ? launch_chains<16>(pb, ch, items, batch, st) : launch_chains<8>(pb, ch, items, batch, st);
+            if (e != hipSuccess) return e;
+        }
+    }
     // 512-thread bound: at most 256 VGPRs per lane and two waves per SIMD.
     // (16 FP64 rows spill a few registers there; measured faster than the
     // spill-free 256-thread bound, which leaves one wave per SIMD.)
@@ -709,29 +751,23 @@ static hipError_t launch_tri_nr(const Prob &pb, int n, long nmodes, int batch, i
         hipError_t e = hipFuncSetAttribute((const void *)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         if (e != hipSuccess) return e;
     }
-    const int per_op = (batch + nop - 1) / nop;
-    const int groups = (per_op + NR - 1) / NR;
-    // grid y holds at most 65535 blocks: launch the right-hand-side groups in
-    // slices, the last slice first (the kernel walks its groups backwards too)
-    if (nop > 65535) return hipErrorInvalidValue;
-    const int gmax = 65535 / nop;
-    for (int g0 = ((groups - 1) / gmax) * gmax; g0 >= 0; g0 -= gmax) {
+    for (int g0 = g_first; g0 >= 0; g0 -= gmax) {
         const int ng = groups - g0 < gmax ? groups - g0 : gmax;
-        dim3 grid((unsigned)((nmodes + W - 1) / W), (unsigned)(nop * ng));
-        hipLaunchKernelGGL(kfn, grid, dim3(threads), shm, st, pb, nmodes, W, P, batch, nop, g0);
+        hipLaunchKernelGGL(kfn, dim3(gx, (unsigned)(ch.rows + nop * ng)), dim3(threads), shm, st, pb, nmodes, W, P, batch, nop,
+                           g0, ch);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
+        ch.rows = 0;   // the chains ride with the first slice
     }
     return hipSuccess;
 }
 
 template <typename T, int MM, class Prob>
-static hipError_t launch_tri_prob(const Prob &pb, int n, long nmodes, int batch, int nop, int W, int P, int nr,
-                                  hipStream_t st) {
-    if (nr == 1) return launch_tri_nr<T, MM, 1>(pb, n, nmodes, batch, nop, W, P, st);
+static hipError_t launch_tri_prob(const Prob &pb, const TriHelm &t, hipStream_t st) {
+    if (t.nr == 1) return launch_tri_nr<T, MM, 1>(pb, t, st);
     if constexpr (sizeof(T) == 8) {   // several right-hand sides per thread: FP64 elimination only
-        if (nr == 2) return launch_tri_nr<T, MM, 2>(pb, n, nmodes, batch, nop, W, P, st);
-        if (nr == 4) return launch_tri_nr<T, MM, 4>(pb, n, nmodes, batch, nop, W, P, st);
+        if (t.nr == 2) return launch_tri_nr<T, MM, 2>(pb, t, st);
+        if (t.nr == 4) return launch_tri_nr<T, MM, 4>(pb, t, st);
     }
     return hipErrorInvalidValue;
 }
@@ -795,7 +831,7 @@ static hipError_t launch_tri_r(const TriHelm &t, const void *in, void *out, hipS
     pb.fwords = t.fwords;
     pb.uni = t.uni;
     if (t.tiled && ((t.tiled & (t.tiled - 1)) || t.tiled % t.W)) return hipErrorInvalidValue;
-    return launch_tri_prob<T, MM>(pb, pb.bands.n, nmodes, t.batch, pb.bands.nop, t.W, t.P, t.nr, st);
+    return launch_tri_prob<T, MM>(pb, t, st);
 }
 
 template <typename T, typename Ti, typename To, int MM>
@@ -812,95 +848,6 @@ static hipError_t launch_tri_mm(const TriHelm &t, const void *in, void *out, hip
     case 16: return launch_tri_t<T, Ti, To, 16>(t, in, out, st);
     default: return hipErrorInvalidValue;
     }
-}
-
-template <int R, int C, typename Ti, typename To, int DIM, bool REAL>
-static hipError_t launch_seq_rc(const TriHelm &t, const void *in, void *out, hipStream_t st) {
-    using OT = typename std::conditional<REAL, double, double2>::type;
-    HelmProb<double, Ti, To, DIM, REAL> pb;
-    pb.bands.Nx = t.Nx;
-    pb.bands.coef = (const double2 *)(REAL ? t.coefr : t.coef);
-    pb.bands.nop = t.nop > 0 ? t.nop : 1;
-    pb.bands.cstride = REAL ? t.cstride / 2 : t.cstride;
-    pb.bands.lamx = t.lamx;
-    pb.bands.lamy = t.lamy;
-    pb.in = (const C2<Ti> *)in;
-    pb.out = (C2<To> *)out;
-    pb.field = t.field;
-    if (t.dim == 2) { pb.bands.n = t.Ny; pb.nmodes = t.Nx; pb.S = t.Nx; }
-    else { pb.bands.n = t.Nz; pb.nmodes = (long)t.Nx * t.Ny; pb.S = (long)t.Nx * t.Ny; }
-    pb.tw = t.tiled;
-    pb.fbits = nullptr;
-    pb.fwords = 0;
-    pb.uni = nullptr;
-    const int n = pb.bands.n;
-    constexpr int PW = 64 / C;
-    const int G = ((n + R - 1) / R + PW - 1) / PW * PW;   // positions, whole waves
-    const int NT = G * C;
-    if (NT > 512) return hipErrorInvalidValue;
-    const long items = (long)t.nfx * t.batch;
-    // Real factors: one chain per part (k_tri_seq_re) when the doubled grid
-    // still runs as one wave of blocks, one block per CU (a block holds a
-    // CU's registers); otherwise one chain per item.  C2's 1152 items: the
-    // split grid's 288 blocks ran in two rounds, 79.6 against 64 us.
-    int ncu = 0;
-    if constexpr (REAL) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            ncu = 0;
-    }
-    if (REAL && (2 * items + C - 1) / C <= ncu) {   // two chains per item: its real and imaginary parts
-        const long blocks = (2 * items + C - 1) / C;
-        hipLaunchKernelGGL((k_tri_seq_re<R, C, DIM == 2, HelmProb<double, Ti, To, DIM, REAL>>), dim3((unsigned)blocks),
-                           dim3(NT), 0, st, pb, t.foff, t.fmode, (const double *)t.fac, t.nent, t.nfx, t.batch,
-                           pb.bands.nop);
-    } else {
-        const long blocks = (items + C - 1) / C;
-        if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((k_tri_seq<R, C, DIM == 2, HelmProb<double, Ti, To, DIM, REAL>, OT>), dim3((unsigned)blocks),
-                           dim3(NT), 0, st, pb, t.foff, t.fmode, (const OT *)t.fac, t.nent, t.nfx, t.batch, pb.bands.nop);
-    }
-    return hipGetLastError();
-}
-
-// As many chains per block as 512 threads hold with R rows per lane.
-template <int R, typename Ti, typename To, int DIM, bool REAL>
-static hipError_t launch_seq_R(const TriHelm &t, const void *in, void *out, hipStream_t st) {
-    const int n = t.dim == 2 ? t.Ny : t.Nz;
-    const int g = (n + R - 1) / R;   // positions of one chain
-    auto fits = [&](int C) { const int PW = 64 / C; return ((g + PW - 1) / PW * PW) * C <= 512; };
-    if (fits(64)) return launch_seq_rc<R, 64, Ti, To, DIM, REAL>(t, in, out, st);
-    if (fits(32)) return launch_seq_rc<R, 32, Ti, To, DIM, REAL>(t, in, out, st);
-    if (fits(16)) return launch_seq_rc<R, 16, Ti, To, DIM, REAL>(t, in, out, st);
-    if (fits(8)) return launch_seq_rc<R, 8, Ti, To, DIM, REAL>(t, in, out, st);
-    if (fits(4)) return launch_seq_rc<R, 4, Ti, To, DIM, REAL>(t, in, out, st);
-    if (fits(2)) return launch_seq_rc<R, 2, Ti, To, DIM, REAL>(t, in, out, st);
-    if (fits(1)) return launch_seq_rc<R, 1, Ti, To, DIM, REAL>(t, in, out, st);
-    return hipErrorInvalidValue;
-}
-
-// 16 rows per lane with real factors; 8 with complex ones (twice the
-// registers), except above n = 4096 where 512 threads need 16
-template <typename Ti, typename To, int DIM, bool REAL>
-static hipError_t launch_seq_d(const TriHelm &t, const void *in, void *out, hipStream_t st) {
-    const int n = t.dim == 2 ? t.Ny : t.Nz;
-    if (REAL || n > 4096) return launch_seq_R<16, Ti, To, DIM, REAL>(t, in, out, st);
-    return launch_seq_R<8, Ti, To, DIM, REAL>(t, in, out, st);
-}
-
-template <typename Ti, typename To>
-static hipError_t launch_seq_t(const TriHelm &t, const void *in, void *out, hipStream_t st) {
-    if (t.dim == 2) return t.real ? launch_seq_d<Ti, To, 2, true>(t, in, out, st) : launch_seq_d<Ti, To, 2, false>(t, in, out, st);
-    return t.real ? launch_seq_d<Ti, To, 3, true>(t, in, out, st) : launch_seq_d<Ti, To, 3, false>(t, in, out, st);
-}
-
-hipError_t launch_tri_seq(const TriHelm &t, DstTypes ty, const void *in, void *out, hipStream_t st) {
-    if (t.nfx <= 0) return hipSuccess;
-    if (!t.foff || !t.fmode || !t.fac || t.batch < 1) return hipErrorInvalidValue;
-    if (ty.in == 0 && ty.out == 0) return launch_seq_t<double, double>(t, in, out, st);
-    if (ty.in == 1 && ty.out == 1) return launch_seq_t<float, float>(t, in, out, st);
-    return hipErrorInvalidValue;
 }
 
 hipError_t launch_tri_helm(const TriHelm &t, DstTypes ty, const void *in, void *out, hipStream_t st) {
