@@ -308,19 +308,43 @@ static int dst_algo_for(const hh_context *c, int N) {
     return 0;
 }
 
-// Block size of the automatic choice: one-wave blocks (one line each) for
-// contiguous rows of N+1 >= 512, measured 3-8% faster there (N+1 = 512: 446
-// against 484 us per GB of rows; 1024: 496 against 521) and slower at 256;
-// 256-thread blocks for strided lines, whose tiles they widen; in FP32,
-// 512-thread blocks (tiles of 32 lines at N+1 = 256: 69 against 74 us per
-// 255^3 pass; in FP64 such a tile's LDS leaves one block per CU and it is
-// slower, 120 against 116 us).
+// Block size of the automatic choice (the blocks compute the same bits): 64,
+// 256 or 512 threads, by the number nb of 256-thread blocks the lines fill.
+//
+// Rows (microseconds per pass, 64 against 256 threads): small one-wave blocks
+// spread a small grid over four times as many CUs and wait for no other wave
+// at their barriers: 6.0 against 9.4 (63 x 63, nb = 1), 7.8 against 10.0 (255
+// rows of 255 x 6, nb = 96), 8.9 against 10.8 (511 x 511 x 2, nb = 128); their
+// smaller LDS lets more of them share a CU in a large one: 47 against 82
+// (63 x 63 x 2048), 40 against 43 (255 x 127 x 200), 99 against 109 (255^3),
+// 414 against 460 (1023 x 1023 x 64).  Where one 256-thread block falls on
+// each CU the larger block is better from N+1 = 128 on: 14 against 17.5 (1023
+// rows of 1023), 11.0 against 12.8 (127 x 127 x 64), with a tie at both ends
+// of the range taken (191 and 319 blocks).  In FP32 a 256-thread block's LDS
+// is already half as large and above N+1 = 128 only the small grids gain:
+// 8.4 against 9.4 (255 x 255 x 8, nb = 128), but 136 against 116 (255^3).
+//
+// Strided lines: the block's width is its segment of a row, so 64 threads pay
+// only where the grid leaves half of the CUs idle and a segment is still 16
+// lines or more (N+1 <= 64): 9.0 against 11.6 (63^3, nb = 63) but 15.8 against
+// 13.4 at nb = 200.  FP32 takes 512 threads at N+1 = 256 (57 against 76 per
+// 255^3 pass; in FP64 such a tile leaves one block per CU and it is slower),
+// and at 128 where the wide tiles fill the chip once (17.2 against 19.3 at
+// 255 x 127 x 63; 14.2 against 12.4 with half of the CUs idle, 35 against 31
+// in two rounds at 255 x 127 x 200).
 static int dst_algo_lines(const hh_context *c, const hh::Lines &ln, int tc) {
-    int algo = dst_algo_for(c, ln.N);
-    // one-wave blocks pay for FP64 rows only (N+1 = 1024: 472 against 521 us); with FP32 storage
-    // 256-thread blocks stay faster (352 against 393 us per pass at 1023^2 x 64)
-    if (c->dst_algo < 0 && !tc && ln.elem_stride == 1 && !ln.in_tw && !ln.out_tw && ln.N + 1 >= 512) algo |= 2;
-    if (c->dst_algo < 0 && ln.elem_stride != 1 && tc && ln.N + 1 >= 128 && ln.N + 1 <= 256) algo |= 4;
+    const int algo = dst_algo_for(c, ln.N), M = ln.N + 1;
+    if (c->dst_algo >= 0 || ln.in_tw || ln.out_tw) return algo;   // mode-tiled rows: a block's lines share segments
+    const long per = M > 16 ? std::max(1, 4096 / M) : 256;   // lines of a 256-thread block
+    if (ln.elem_stride == 1) {
+        const long nb = (ln.ncols * ln.nplanes + per - 1) / per;
+        if (M <= 64) return algo | 2;
+        if (tc) return M <= 128 || nb <= 192 ? algo | 2 : algo;
+        return nb > 192 && nb < 320 ? algo : algo | 2;
+    }
+    const long nb = (ln.ncols + per - 1) / per * ln.nplanes;
+    if (M <= 64) return nb < 128 ? algo | 2 : algo;
+    if (tc && (M == 256 || (M == 128 && nb > 448 && nb <= 1024))) return algo | 4;
     return algo;
 }
 
