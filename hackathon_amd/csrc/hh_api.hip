@@ -64,7 +64,11 @@ struct hh_context {
     int dst_algo = -1;                  // -1 auto; bit 0: odd extension (else (N+1)-point), bit 1: 64-thread blocks
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
-    double *d_norm = nullptr;
+    double *d_norm = nullptr;           // per-block norms, then the residuals' maxima (zero between solves)
+    // their two results, in host memory that the kernels write: copied from the
+    // device they cost a refinement 28 us more per sweep
+    double *h_norm = nullptr;
+    void *residual_slots() const { return d_norm + 2 * hh::NORM_BLOCKS; }
     size_t budget = 0, in_use = 0;
     void *noalloc_ws = nullptr;         // this device's noalloc_scratch (device address)
     hipError_t noalloc_status = hipSuccess;
@@ -426,7 +430,11 @@ extern "C" int hh_context_create(int device, hh_context **out) {
         c->noalloc_ws = it->second.first;
         c->noalloc_status = it->second.second;
     }
-    if (hipMalloc((void **)&c->d_norm, hh::norm_buffer_doubles() * sizeof(double)) != hipSuccess) {
+    const std::vector<double> zeros(2 * hh::NORM_SLOTS, 0.0);
+    if (hipMalloc((void **)&c->d_norm, 2 * (hh::NORM_BLOCKS + hh::NORM_SLOTS) * sizeof(double)) != hipSuccess ||
+        hipMemcpy(c->residual_slots(), zeros.data(), zeros.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
+        hipHostMalloc((void **)&c->h_norm, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        (void)hipFree(c->d_norm);
         (void)hipStreamDestroy(c->own);
         delete c;
         return fail(HH_ERR_NOMEM, "norm buffer allocation failed");
@@ -449,6 +457,7 @@ extern "C" int hh_context_destroy(hh_context *c) {
     for (auto &r : c->recs) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
     for (auto e : c->pool) (void)hipEventDestroy(e);
     (void)hipFree(c->d_norm);
+    (void)hipHostFree(c->h_norm);
     (void)hipStreamDestroy(c->own);
     delete c;
     return HH_OK;
@@ -1319,23 +1328,33 @@ static int solve_core(hh_plan *p, int ti, int tc, int to, int tri_comp, const vo
     return dst_pass(c, lx, tc, tc, to, ws, sol, acc);
 }
 
-static int residual_into(hh_plan *p, const void *u, const void *F, void *res, int res_f32, int batch) {
-    TimeScope ts(p->ctx, 3, (double)hh_plan_field_size(p) * batch * (32 + (res_f32 ? 8 : 16)));
-    hipError_t e;
-    if (p->dim == 2)
-        e = hh::launch_residual2d(p->Nx, p->Ny, batch, p->coef64, p->nop, u, F, res, res_f32, p->ctx->stream);
-    else
-        e = hh::launch_residual3d(p->Nx, p->Ny, p->Nz, batch, p->coef64, p->nop, u, F, res, res_f32, p->ctx->stream);
-    if (e != hipSuccess) return fail(HH_ERR_DEVICE, "residual launch failed: %s", hipGetErrorString(e));
+static int read_norms(hh_context *c, double out[2]) {
+    HIPCHK(hipStreamSynchronize(c->stream));
+    out[0] = c->h_norm[0];
+    out[1] = c->h_norm[1];
     return HH_OK;
 }
 
-static int norms_sync(hh_context *c, long n, const void *x, int x_f32, const void *y, double out[2], bool l2 = false) {
-    hipError_t e = hh::launch_norms(n, x, x_f32, y, c->d_norm, c->stream, l2);
+// norms (FP32 results): norms[0..1] = max |res| and max |F|, waited for.
+static int residual_into(hh_plan *p, const void *u, const void *F, void *res, int res_f32, int batch,
+                         double *norms = nullptr) {
+    TimeScope ts(p->ctx, 3, (double)hh_plan_field_size(p) * batch * (32 + (res_f32 ? 8 : 16)));
+    hh_context *c = p->ctx;
+    void *slots = norms ? c->residual_slots() : nullptr;
+    hipError_t e;
+    if (p->dim == 2)
+        e = hh::launch_residual2d(p->Nx, p->Ny, batch, p->coef64, p->nop, u, F, res, res_f32, slots, c->stream);
+    else
+        e = hh::launch_residual3d(p->Nx, p->Ny, p->Nz, batch, p->coef64, p->nop, u, F, res, res_f32, slots, c->stream);
+    if (e == hipSuccess && norms) e = hh::launch_residual_norms(slots, c->h_norm, c->stream);
+    if (e != hipSuccess) return fail(HH_ERR_DEVICE, "residual launch failed: %s", hipGetErrorString(e));
+    return norms ? read_norms(c, norms) : HH_OK;
+}
+
+static int norms_sync(hh_context *c, long n, const void *x, const void *y, double out[2], bool l2 = false) {
+    hipError_t e = hh::launch_norms(n, x, y, c->d_norm, c->h_norm, c->stream, l2);
     if (e != hipSuccess) return fail(HH_ERR_DEVICE, "norm launch failed: %s", hipGetErrorString(e));
-    HIPCHK(hipMemcpyAsync(out, c->d_norm, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return HH_OK;
+    return read_norms(c, out);
 }
 
 // HH_ERR_SINGULAR when an operator that right-hand sides 0..batch-1 use is
@@ -1384,17 +1403,14 @@ static int solve_ws(hh_plan *p, const void *rhs, void *sol, int batch, void *scr
         p->last_rel = -1.0;
         return HH_OK;
     }
-    double nf[2], nr[2];
-    if ((rc = norms_sync(c, n, rhs, 0, nullptr, nf))) return rc;
-    const double fn = nf[0] > 0 ? nf[0] : 1.0;
     int sweeps = 0;
     double rel = 0;
     for (;;) {
         // r = A u - F with FP64 arithmetic, stored in FP32 (its norm only
         // needs a few digits; the correction it drives is an FP32 solve)
-        if ((rc = residual_into(p, sol, rhs, dlt, 1, batch))) return rc;
-        if ((rc = norms_sync(c, n, dlt, 1, nullptr, nr))) return rc;
-        rel = nr[0] / fn;
+        double nrf[2];   // max |r|, max |F|
+        if ((rc = residual_into(p, sol, rhs, dlt, 1, batch, nrf))) return rc;
+        rel = nrf[0] / (nrf[1] > 0 ? nrf[1] : 1.0);
         if (rel <= p->tol || sweeps >= p->max_iter) break;
         if ((rc = solve_core(p, 1, 1, 0, 1, dlt, sol, tws, batch, -1.0))) return rc;   // u -= A32^{-1} r
         sweeps++;
@@ -1775,7 +1791,7 @@ extern "C" int hh_norms(hh_context *c, long n, const void *x, const void *y, dou
     std::lock_guard<std::mutex> lk(c->mu);
     int rc = set_device(c);
     if (rc) return rc;
-    return norms_sync(c, n, x, 0, y, out);
+    return norms_sync(c, n, x, y, out);
 }
 
 extern "C" int hh_norms_l2(hh_context *c, long n, const void *x, const void *y, double out[2]) {
@@ -1784,5 +1800,5 @@ extern "C" int hh_norms_l2(hh_context *c, long n, const void *x, const void *y, 
     std::lock_guard<std::mutex> lk(c->mu);
     int rc = set_device(c);
     if (rc) return rc;
-    return norms_sync(c, n, x, 0, y, out, true);
+    return norms_sync(c, n, x, y, out, true);
 }

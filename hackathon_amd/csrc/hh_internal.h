@@ -152,21 +152,21 @@ struct Rhs3D {
 hipError_t launch_rhs3d(const Rhs3D &r, void *F, hipStream_t st);
 hipError_t launch_rhs3d_6(const Rhs3D &r, void *F, hipStream_t st);   // sixth order (hh_compact.hip)
 
-// res = A u - F (the reference residual.c), and the fused refinement pieces.
+// res = A u - F (the reference residual.c).
 // coef tables: right-hand side b uses coef + (b % nop) * (6 Ny | 12 Nz)
+// norms (null: none; FP32 results only): 2 NORM_SLOTS words, zero, that gather
+// the maxima of |res|^2 and |F|^2; launch_residual_norms roots them into
+// out[0..1] and zeroes the words again.
+constexpr int NORM_SLOTS = 256;
 hipError_t launch_residual2d(int Nx, int Ny, int batch, const void *coef, int nop, const void *u,
-                             const void *F, void *res, int res_f32, hipStream_t st);
+                             const void *F, void *res, int res_f32, void *norms, hipStream_t st);
 hipError_t launch_residual3d(int Nx, int Ny, int Nz, int batch, const void *coef, int nop, const void *u,
-                             const void *F, void *res, int res_f32, hipStream_t st);
-// u += s*c (c in FP32 or FP64)
-hipError_t launch_axpy_update(long n, void *u, const void *c, int c_f32, double s, hipStream_t st);
-// out[0] = max |x|, out[1] = max |x - y| (y may be null); out is device
-// memory of norm_buffer_doubles() values, out[2..] the per-block partials
+                             const void *F, void *res, int res_f32, void *norms, hipStream_t st);
+hipError_t launch_residual_norms(void *norms, double *out, hipStream_t st);
+// out[0..1] = the max norms (l2: the 2-norms) of x and x - y (y may be null);
+// part: device memory of 2 NORM_BLOCKS values for the per-block results
 constexpr int NORM_BLOCKS = 2048;
-constexpr long norm_buffer_doubles() { return 2 + 2L * NORM_BLOCKS; }
-// out[0..1] = the max norms (l2: the 2-norms) of x and x - y; out[2..] scratch
-hipError_t launch_norms(long n, const void *x, int x_f32, const void *y, double *out, hipStream_t st,
+hipError_t launch_norms(long n, const void *x, const void *y, double *part, double *out, hipStream_t st,
                         bool l2 = false);
-hipError_t launch_convert(long n, const void *in, int in_f32, void *out, int out_f32, hipStream_t st);
 
 }  // namespace hh

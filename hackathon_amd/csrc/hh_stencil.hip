@@ -132,14 +132,39 @@ hipError_t launch_rhs3d(const Rhs3D &r, void *F, hipStream_t st) {
 // 64 x 1023^2: 689 -> 599 us (5.4 TB/s), 8 x 1023^2: 93 -> 74 us.
 constexpr int RES_ROWS = 4;   // rows per thread in 2D (8 rows: 618 and 79 us; 16: 663 and 92)
 
-template <typename To>
-__global__ __launch_bounds__(256) void k_residual2d(int Nx, int Ny, int nchunk, const z2 *__restrict__ coef, int nop, const z2 *u,
-                                                    const z2 *F, C2<To> *res, int b0) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
+// NORM: the maxima of |res|^2 (as stored) and |F|^2 go to `norms` as well, one
+// atomic maximum of each per block (the bits of a nonnegative double order as
+// an integer, so the result does not depend on the order).  A refinement
+// sweep's norm then costs no pass of its own: 127 x 255 x 200 in FP32, 11 us a
+// sweep, and 17 us for the norm of F.
+template <int NT> HH_DEV void block_norms(double r2, double f2, unsigned long long *norms, unsigned block) {
+    constexpr int NW = NT / 64;
+    __shared__ double part[2 * NW];
+    const int t = threadIdx.y * blockDim.x + threadIdx.x;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) {
+        r2 = fmax(r2, __shfl_xor(r2, s));
+        f2 = fmax(f2, __shfl_xor(f2, s));
+    }
+    if (t % 64 == 0) { part[t / 64] = r2; part[NW + t / 64] = f2; }
+    __syncthreads();
+    if (t < 2) {
+        double m = part[t * NW];
+#pragma unroll
+        for (int k = 1; k < NW; k++) m = fmax(m, part[t * NW + k]);
+        atomicMax(norms + t * NORM_SLOTS + block % NORM_SLOTS, (unsigned long long)__double_as_longlong(m));
+    }
+}
+
+template <typename To, bool NORM>
+__global__ __launch_bounds__(256) void k_residual2d(int Nx, int Ny, const z2 *__restrict__ coef, int nop, const z2 *u,
+                                                    const z2 *F, C2<To> *res, int b0, unsigned long long *norms) {
+    int i = blockIdx.x * 256 + threadIdx.x;
     const int j0 = blockIdx.y * RES_ROWS;
     const int b = b0 + (int)blockIdx.z;
-    if (i >= Nx) return;
-    (void)nchunk;
+    double r2 = 0, f2 = 0;
+    if constexpr (NORM) i = min(i, Nx - 1);   // idle lanes repeat the last column
+    else if (i >= Nx) return;
     const long Nxy = (long)Nx * Ny;
     const z2 *ub = u + b * Nxy;
     const z2 *cb = coef + 6L * (b % nop) * Ny;   // per row: bm, am, b, a, bp, ap
@@ -161,10 +186,17 @@ __global__ __launch_bounds__(256) void k_residual2d(int Nx, int Ny, int nchunk, 
         const z2 mid = za(za(zm(cq[2], l0), zm(cq[3], c0)), zm(cq[2], r0));
         const z2 bot = za(za(zm(cq[0], lm), zm(cq[1], cm)), zm(cq[0], rm));
         const long id = b * Nxy + (long)j * Nx + i;
-        res[id] = cconv<To, double>(zd(za(za(top, mid), bot), F[id]));
+        const z2 f = F[id];
+        const C2<To> r = cconv<To, double>(zd(za(za(top, mid), bot), f));
+        res[id] = r;
+        if constexpr (NORM) {
+            r2 = fmax(r2, cabs2<double>(cconv<double, To>(r)));
+            f2 = fmax(f2, cabs2<double>(f));
+        }
         lm = l0; cm = c0; rm = r0;
         l0 = lp; c0 = cp; r0 = rp;
     }
+    if constexpr (NORM) block_norms<256>(r2, f2, norms, blockIdx.y + blockIdx.z * gridDim.y);
 }
 
 
@@ -184,9 +216,10 @@ __global__ __launch_bounds__(256) void k_residual2d(int Nx, int Ny, int nchunk, 
 // fewer idle lanes (200^3: 89 against 95 us; 255^3: 178 against 168).
 constexpr int RY = 8, RZ = 16;
 
-template <typename To, int RX>
+template <typename To, int RX, bool NORM>
 __global__ __launch_bounds__(RX * RY) void k_residual3d(int Nx, int Ny, int Nz, int nchunk, const z2 *__restrict__ coef, int nop,
-                                                       const z2 *u, const z2 *F, C2<To> *res, int b0) {
+                                                       const z2 *u, const z2 *F, C2<To> *res, int b0,
+                                                       unsigned long long *norms) {
     constexpr int HX = RX + 2, HY = RY + 2, HE = HX * HY, NT = RX * RY;
     static_assert(HE <= 2 * NT, "a layer tile with halo takes at most two loads per thread");
     __shared__ z2 lay[3][HE];
@@ -249,6 +282,7 @@ __global__ __launch_bounds__(RX * RY) void k_residual3d(int Nx, int Ny, int Nz, 
     Part pm, pc, pp;
     plane(0, pm);
     plane(1, pc);
+    double r2 = 0, f2 = 0;
     int sn = 2;   // the slot of layer l+1: that of layer l-2, last read a barrier ago
     for (int l = l0; l < l1; l++) {
         stash(sn, l + 1);
@@ -263,7 +297,12 @@ __global__ __launch_bounds__(RX * RY) void k_residual3d(int Nx, int Ny, int Nz, 
             z2 acc = layer(pm, cl + 8);
             acc = za(acc, layer(pc, cl));
             acc = za(acc, layer(pp, cl + 4));
-            res[id0 + (long)l * Nxy] = cconv<To, double>(zd(acc, f));
+            const C2<To> r = cconv<To, double>(zd(acc, f));
+            res[id0 + (long)l * Nxy] = r;
+            if constexpr (NORM) {
+                r2 = fmax(r2, cabs2<double>(cconv<double, To>(r)));
+                f2 = fmax(f2, cabs2<double>(f));
+            }
         }
         pm = pc;
         pc = pp;
@@ -271,72 +310,48 @@ __global__ __launch_bounds__(RX * RY) void k_residual3d(int Nx, int Ny, int Nz, 
         // the next step's barrier, after its read here, by then
         sn = sn == 2 ? 0 : sn + 1;
     }
+    if constexpr (NORM)
+        block_norms<NT>(r2, f2, norms, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
 }
 
 hipError_t launch_residual2d(int Nx, int Ny, int batch, const void *coef, int nop, const void *u, const void *F,
-                             void *res, int res_f32, hipStream_t st) {
-    const int nchunk = (Ny + RES_ROWS - 1) / RES_ROWS;
+                             void *res, int res_f32, void *norms, hipStream_t st) {
+    if (norms && !res_f32) return hipErrorInvalidValue;
     for (int b0 = 0; b0 < batch; b0 += 65535) {   // grid z holds at most 65535 right-hand sides
         const int nb = batch - b0 < 65535 ? batch - b0 : 65535;
-        dim3 g((unsigned)((Nx + 255) / 256), (unsigned)nchunk, (unsigned)nb);
-        if (res_f32)
-            hipLaunchKernelGGL(k_residual2d<float>, g, dim3(256), 0, st, Nx, Ny, nchunk, (const z2 *)coef, nop,
-                               (const z2 *)u, (const z2 *)F, (float2 *)res, b0);
-        else
-            hipLaunchKernelGGL(k_residual2d<double>, g, dim3(256), 0, st, Nx, Ny, nchunk, (const z2 *)coef, nop,
-                               (const z2 *)u, (const z2 *)F, (z2 *)res, b0);
+        dim3 g((unsigned)((Nx + 255) / 256), (unsigned)((Ny + RES_ROWS - 1) / RES_ROWS), (unsigned)nb);
+        auto run = [&](auto kfn, auto *out) {
+            hipLaunchKernelGGL(kfn, g, dim3(256), 0, st, Nx, Ny, (const z2 *)coef, nop, (const z2 *)u, (const z2 *)F, out,
+                               b0, (unsigned long long *)norms);
+        };
+        if (norms) run(k_residual2d<float, true>, (float2 *)res);
+        else if (res_f32) run(k_residual2d<float, false>, (float2 *)res);
+        else run(k_residual2d<double, false>, (z2 *)res);
     }
     return hipGetLastError();
 }
 
 hipError_t launch_residual3d(int Nx, int Ny, int Nz, int batch, const void *coef, int nop, const void *u,
-                             const void *F, void *res, int res_f32, hipStream_t st) {
+                             const void *F, void *res, int res_f32, void *norms, hipStream_t st) {
     const int nchunk = (Nz + RZ - 1) / RZ;
     const int per = 65535 / nchunk;   // right-hand sides per launch (grid z)
-    if (per < 1) return hipErrorInvalidValue;
+    if (per < 1 || (norms && !res_f32)) return hipErrorInvalidValue;
     const int RX = (Nx + 63) / 64 * 64 > (Nx + 31) / 32 * 32 ? 32 : 64;
     for (int b0 = 0; b0 < batch; b0 += per) {
         const int nb = batch - b0 < per ? batch - b0 : per;
         dim3 g((unsigned)((Nx + RX - 1) / RX), (unsigned)((Ny + RY - 1) / RY), (unsigned)(nchunk * nb));
         auto run = [&](auto kfn, auto *out) {
             hipLaunchKernelGGL(kfn, g, dim3(RX, RY), 0, st, Nx, Ny, Nz, nchunk, (const z2 *)coef, nop, (const z2 *)u,
-                               (const z2 *)F, out, b0);
+                               (const z2 *)F, out, b0, (unsigned long long *)norms);
         };
-        if (res_f32) run(RX == 64 ? k_residual3d<float, 64> : k_residual3d<float, 32>, (float2 *)res);
-        else run(RX == 64 ? k_residual3d<double, 64> : k_residual3d<double, 32>, (z2 *)res);
+        if (norms) run(RX == 64 ? k_residual3d<float, 64, true> : k_residual3d<float, 32, true>, (float2 *)res);
+        else if (res_f32) run(RX == 64 ? k_residual3d<float, 64, false> : k_residual3d<float, 32, false>, (float2 *)res);
+        else run(RX == 64 ? k_residual3d<double, 64, false> : k_residual3d<double, 32, false>, (z2 *)res);
     }
     return hipGetLastError();
 }
 
-// ---------------------------------------------------------------- small ops
-template <typename Tc>
-__global__ void k_update(long n, z2 *u, const C2<Tc> *c, double s) {
-    long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id < n) u[id] = za(u[id], zs(cconv<double, Tc>(c[id]), s));
-}
-
-hipError_t launch_axpy_update(long n, void *u, const void *c, int c_f32, double s, hipStream_t st) {
-    dim3 g((unsigned)((n + 255) / 256));
-    if (c_f32) hipLaunchKernelGGL(k_update<float>, g, dim3(256), 0, st, n, (z2 *)u, (const float2 *)c, s);
-    else hipLaunchKernelGGL(k_update<double>, g, dim3(256), 0, st, n, (z2 *)u, (const z2 *)c, s);
-    return hipGetLastError();
-}
-
-template <typename Ti, typename To>
-__global__ void k_convert(long n, const C2<Ti> *in, C2<To> *out) {
-    long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id < n) out[id] = cconv<To, Ti>(in[id]);
-}
-
-hipError_t launch_convert(long n, const void *in, int in_f32, void *out, int out_f32, hipStream_t st) {
-    dim3 g((unsigned)((n + 255) / 256));
-    if (!in_f32 && out_f32) hipLaunchKernelGGL((k_convert<double, float>), g, dim3(256), 0, st, n, (const z2 *)in, (float2 *)out);
-    else if (in_f32 && !out_f32) hipLaunchKernelGGL((k_convert<float, double>), g, dim3(256), 0, st, n, (const float2 *)in, (z2 *)out);
-    else if (in_f32) hipLaunchKernelGGL((k_convert<float, float>), g, dim3(256), 0, st, n, (const float2 *)in, (float2 *)out);
-    else hipLaunchKernelGGL((k_convert<double, double>), g, dim3(256), 0, st, n, (const z2 *)in, (z2 *)out);
-    return hipGetLastError();
-}
-
+// ---------------------------------------------------------------- norms
 // max |x| and max |x - y| (L2 = false), or sqrt(sum |x|^2) and
 // sqrt(sum |x - y|^2) (L2 = true), over n complex values, in two passes
 // without atomics: each block writes the maxima (sums) of |x|^2 and
@@ -348,8 +363,8 @@ hipError_t launch_convert(long n, const void *in, int in_f32, void *out, int out
 // loaded before any is used.
 template <bool L2> HH_DEV double norm_join(double a, double b) { return L2 ? a + b : fmax(a, b); }
 
-template <typename Tx, bool L2>
-__global__ __launch_bounds__(256) void k_norms(long n, const C2<Tx> *x, const z2 *y, double *part) {
+template <bool L2>
+__global__ __launch_bounds__(256) void k_norms(long n, const z2 *x, const z2 *y, double *part) {
     __shared__ double s0[256], s1[256];
     double m0 = 0, m1 = 0;
     const long stride = (long)gridDim.x * blockDim.x;
@@ -357,7 +372,7 @@ __global__ __launch_bounds__(256) void k_norms(long n, const C2<Tx> *x, const z2
     for (; id + 3 * stride < n; id += 4 * stride) {
         z2 a[4], c[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) a[u] = cconv<double, Tx>(x[id + u * stride]);
+        for (int u = 0; u < 4; u++) a[u] = x[id + u * stride];
         if (y) {
 #pragma unroll
             for (int u = 0; u < 4; u++) c[u] = y[id + u * stride];
@@ -369,7 +384,7 @@ __global__ __launch_bounds__(256) void k_norms(long n, const C2<Tx> *x, const z2
         }
     }
     for (; id < n; id += stride) {
-        const z2 a = cconv<double, Tx>(x[id]);
+        const z2 a = x[id];
         m0 = norm_join<L2>(m0, cabs2<double>(a));
         if (y) m1 = norm_join<L2>(m1, cabs2<double>(zd(a, y[id])));
     }
@@ -413,19 +428,36 @@ __global__ __launch_bounds__(256) void k_norms_final(int nb, const double *part,
     }
 }
 
-hipError_t launch_norms(long n, const void *x, int x_f32, const void *y, double *out, hipStream_t st, bool l2) {
+// The two maxima that the residuals left in `norms`, rooted, which are zeroed for the next sweep.
+static_assert(NORM_SLOTS == 256, "one slot of each maximum per thread");
+__global__ __launch_bounds__(256) void k_residual_norms(unsigned long long *norms, double *out) {
+    __shared__ double part[8];
+    const int t = threadIdx.x;
+    double m[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        m[k] = __longlong_as_double((long long)norms[k * NORM_SLOTS + t]);
+        norms[k * NORM_SLOTS + t] = 0;
+#pragma unroll
+        for (int s = 32; s > 0; s >>= 1) m[k] = fmax(m[k], __shfl_xor(m[k], s));
+        if (t % 64 == 0) part[4 * k + t / 64] = m[k];
+    }
+    __syncthreads();
+    if (t < 2) out[t] = sqrt(fmax(fmax(part[4 * t], part[4 * t + 1]), fmax(part[4 * t + 2], part[4 * t + 3])));
+}
+
+hipError_t launch_residual_norms(void *norms, double *out, hipStream_t st) {
+    hipLaunchKernelGGL(k_residual_norms, dim3(1), dim3(256), 0, st, (unsigned long long *)norms, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_norms(long n, const void *x, const void *y, double *part, double *out, hipStream_t st, bool l2) {
     long blocks = (n + 2047) / 2048;   // about eight values per thread
     if (blocks > NORM_BLOCKS) blocks = NORM_BLOCKS;
     if (blocks < 1) blocks = 1;
-    double *part = out + 2;
     auto run = [&](auto L) -> hipError_t {
         constexpr bool B = decltype(L)::value;
-        if (x_f32)
-            hipLaunchKernelGGL((k_norms<float, B>), dim3((unsigned)blocks), dim3(256), 0, st, n, (const float2 *)x,
-                               (const z2 *)y, part);
-        else
-            hipLaunchKernelGGL((k_norms<double, B>), dim3((unsigned)blocks), dim3(256), 0, st, n, (const z2 *)x,
-                               (const z2 *)y, part);
+        hipLaunchKernelGGL(k_norms<B>, dim3((unsigned)blocks), dim3(256), 0, st, n, (const z2 *)x, (const z2 *)y, part);
         hipLaunchKernelGGL(k_norms_final<B>, dim3(1), dim3(256), 0, st, (int)blocks, (const double *)part, out);
         return hipGetLastError();
     };
