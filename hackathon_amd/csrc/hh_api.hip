@@ -65,9 +65,14 @@ struct hh_context {
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
     double *d_norm = nullptr;           // per-block norms, then the residuals' maxima (zero between solves)
-    // their two results, in host memory that the kernels write: copied from the
-    // device they cost a refinement 28 us more per sweep
+    // their two results, in host memory that the kernels write (copied from the
+    // device they cost a refinement 28 us more per sweep)
     double *h_norm = nullptr;
+    // pinned memory from which the device reads a plan's operator tables, and
+    // the event of its last reader
+    void *stage = nullptr;
+    size_t stage_bytes = 0;
+    hipEvent_t staged = nullptr;
     void *residual_slots() const { return d_norm + 2 * hh::NORM_BLOCKS; }
     size_t budget = 0, in_use = 0;
     void *noalloc_ws = nullptr;         // this device's noalloc_scratch (device address)
@@ -129,12 +134,9 @@ struct hh_plan {
     void *coef64 = nullptr, *coef32 = nullptr;   // [op][q][6] or [op][q][12]
     double *lamx = nullptr, *lamy = nullptr;
     std::vector<cd> hcoef;                       // host copy of the band table
-    std::vector<float> h32;                      // FP32 copy staged for hh_plan_set_operators
     // real parts of the table, same order (read as (re c_2i, re c_2i+1) pairs by
     // the real-band tridiagonal kernels), FP64 and FP32
     void *coefr64 = nullptr, *coefr32 = nullptr;
-    std::vector<double> hr64;
-    std::vector<float> hr32;
     int real_op = 0;                             // every coefficient of the current operators real
     int real_mode = -1;                          // -1: real-band kernels when real_op; 0: complex-band always
     int cap_nop = 1;                             // operator slots allocated on the device
@@ -158,8 +160,6 @@ struct hh_plan {
     std::vector<int2> hent;
     uint32_t *d_bits = nullptr;
     void *d_facc = nullptr, *d_facr = nullptr;
-    std::vector<cd> hfacc_t;                     // staging of the device layout
-    std::vector<double> hfacr_t;
     size_t cap_ent = 0, cap_bits = 0, cap_facc = 0, cap_facr = 0;
     // Generation: bumped whenever a change would invalidate a recorded graph
     // (device tables reallocated, band kind, operator count or launch shapes
@@ -433,7 +433,9 @@ extern "C" int hh_context_create(int device, hh_context **out) {
     const std::vector<double> zeros(2 * hh::NORM_SLOTS, 0.0);
     if (hipMalloc((void **)&c->d_norm, 2 * (hh::NORM_BLOCKS + hh::NORM_SLOTS) * sizeof(double)) != hipSuccess ||
         hipMemcpy(c->residual_slots(), zeros.data(), zeros.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-        hipHostMalloc((void **)&c->h_norm, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void **)&c->h_norm, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess ||
+        hipEventCreateWithFlags(&c->staged, hipEventDisableTiming) != hipSuccess) {
+        (void)hipHostFree(c->h_norm);
         (void)hipFree(c->d_norm);
         (void)hipStreamDestroy(c->own);
         delete c;
@@ -458,6 +460,9 @@ extern "C" int hh_context_destroy(hh_context *c) {
     for (auto e : c->pool) (void)hipEventDestroy(e);
     (void)hipFree(c->d_norm);
     (void)hipHostFree(c->h_norm);
+    (void)hipEventSynchronize(c->staged);
+    (void)hipHostFree(c->stage);
+    (void)hipEventDestroy(c->staged);
     (void)hipStreamDestroy(c->own);
     delete c;
     return HH_OK;
@@ -734,19 +739,6 @@ extern "C" int hh_robin3d(int Nx, int Ny, int Nz, double h, const double *alpha_
 // Device band-table order from the caller's operator vectors.
 // 2D: input [op][bp, ap, b, a, bm, am][Ny] -> table [op][q](bm, am, b, a, bp, ap);
 // 3D: input [op][a..dm][Nz] -> table [op][l][12].
-static void fill_real(hh_plan *p) {
-    const size_t cnt = p->hcoef.size();
-    p->hr64.resize(cnt);
-    p->hr32.resize(cnt);
-    int real = 1;
-    for (size_t i = 0; i < cnt; i++) {
-        p->hr64[i] = p->hcoef[i].real();
-        p->hr32[i] = (float)p->hcoef[i].real();
-        if (p->hcoef[i].imag() != 0.0) real = 0;
-    }
-    p->real_op = real;
-}
-
 static void build_table(int dim, int n, int nop, const double *coef, std::vector<cd> &tab) {
     if (dim == 2) {
         static const int src[6] = {4, 5, 2, 3, 0, 1};
@@ -764,9 +756,15 @@ static void build_table(int dim, int n, int nop, const double *coef, std::vector
     }
 }
 
+static bool table_real(const std::vector<cd> &tab) {
+    for (const cd &v : tab)
+        if (v.imag() != 0.0) return false;
+    return true;
+}
+
 static void fill_table(hh_plan *p, int nop, const double *coef) {
     build_table(p->dim, p->dim == 2 ? p->Ny : p->Nz, nop, coef, p->hcoef);
-    fill_real(p);
+    p->real_op = table_real(p->hcoef);
     hh::classify_modes(p->dim, p->Nx, p->Ny, p->Nz, nop, p->hcoef.data(), p->hlamx.data(), p->hlamy.data(),
                        p->real_op != 0, p->kappa_flag, p->ms);
 }
@@ -801,40 +799,62 @@ static int ensure_dev(hh_plan *p, void **ptr, size_t *cap, size_t bytes) {
     return HH_OK;
 }
 
-// Copies the near-resonant mode tables to the device, stream-ordered after
-// the work already queued (the host vectors stay untouched until the next
-// fill_table, which waits for the stream first).
-static int upload_modes(hh_plan *p) {
+// The device tables of the plan's operators (nop of them in hcoef and ms) from
+// the host's, stream-ordered after the work already queued; the context's lock
+// is held.
+static int upload_tables(hh_plan *p) {
     hh_context *c = p->ctx;
-    hh::ModeSet &m = p->ms;
+    const hh::ModeSet &m = p->ms;
+    const size_t ne = m.fmode.size(), nf = ne * m.n * 4;
     int rc;
-    // device layout of the factors: [row][entry](L, P, R, Up), so that the
-    // lanes of neighbouring entries read neighbouring records
-    const long ne = (long)m.fmode.size(), n = m.n;
-    p->hfacc_t.resize(m.facc.size());
-    p->hfacr_t.resize(m.facr.size());
-    for (long e = 0; e < ne; e++)
-        for (long q = 0; q < n; q++)
-            for (int k = 0; k < 4; k++) {
-                p->hfacc_t[(q * ne + e) * 4 + k] = m.facc[(e * n + q) * 4 + k];
-                if (!m.facr.empty()) p->hfacr_t[(q * ne + e) * 4 + k] = m.facr[(e * n + q) * 4 + k];
-            }
     // one row of nfx entries per operator, padded with (-1, 0)
     p->hent.assign((size_t)m.nop * m.nfx, make_int2(-1, 0));
     for (int o = 0; o < m.nop; o++)
         for (int e = m.foff[o]; e < m.foff[o + 1]; e++) p->hent[(size_t)o * m.nfx + e - m.foff[o]] = make_int2(m.fmode[e], e);
     if ((rc = ensure_dev(p, (void **)&p->d_ent, &p->cap_ent, p->hent.size() * sizeof(int2)))) return rc;
     if ((rc = ensure_dev(p, (void **)&p->d_bits, &p->cap_bits, m.bits.size() * sizeof(uint32_t)))) return rc;
-    if ((rc = ensure_dev(p, &p->d_facc, &p->cap_facc, m.facc.size() * sizeof(cd)))) return rc;
-    if ((rc = ensure_dev(p, &p->d_facr, &p->cap_facr, m.facr.size() * sizeof(double)))) return rc;
-    auto cp = [&](void *d, const void *h, size_t bytes) -> int {
-        if (bytes) HIPCHK(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, c->stream));
-        return HH_OK;
-    };
-    if ((rc = cp(p->d_ent, p->hent.data(), p->hent.size() * sizeof(int2)))) return rc;
-    if ((rc = cp(p->d_bits, m.bits.data(), m.bits.size() * sizeof(uint32_t)))) return rc;
-    if ((rc = cp(p->d_facc, p->hfacc_t.data(), p->hfacc_t.size() * sizeof(cd)))) return rc;
-    return cp(p->d_facr, p->hfacr_t.data(), p->hfacr_t.size() * sizeof(double));
+    if ((rc = ensure_dev(p, &p->d_facc, &p->cap_facc, nf * sizeof(cd)))) return rc;
+    if ((rc = ensure_dev(p, &p->d_facr, &p->cap_facr, (p->real_op ? nf : 0) * sizeof(double)))) return rc;
+    // staging: bands, factors, entries, bits (each a multiple of 16 bytes)
+    const void *src[4] = {p->hcoef.data(), p->real_op ? (const void *)m.facr.data() : (const void *)m.facc.data(),
+                          p->hent.data(), m.bits.data()};
+    const size_t len[4] = {p->hcoef.size() * sizeof(cd), nf * (p->real_op ? sizeof(double) : sizeof(cd)),
+                           p->hent.size() * sizeof(int2), m.bits.size() * sizeof(uint32_t)};
+    size_t at[4], total = 0;
+    for (int k = 0; k < 4; k++) { at[k] = total; total += (len[k] + 15) / 16 * 16; }
+    HIPCHK(hipEventSynchronize(c->staged));
+    if (total > c->stage_bytes) {
+        const size_t want = std::max(total + total / 2, (size_t)256 << 10);
+        (void)hipHostFree(c->stage);
+        c->stage = nullptr;
+        c->stage_bytes = 0;
+        if (hipHostMalloc(&c->stage, want, hipHostMallocDefault) != hipSuccess)
+            return fail(HH_ERR_NOMEM, "pinned allocation of %zu bytes failed", want);
+        c->stage_bytes = want;
+    }
+    char *base = (char *)c->stage;
+    for (int k = 0; k < 4; k++)
+        if (len[k]) memcpy(base + at[k], src[k], len[k]);
+    hh::OperatorTables t;
+    t.ncoef = (long)p->hcoef.size();
+    t.coef = (const double2 *)(base + at[0]);
+    t.coef64 = (double2 *)p->coef64; t.coef32 = (float2 *)p->coef32;
+    t.coefr64 = (double *)p->coefr64; t.coefr32 = (float *)p->coefr32;
+    t.n = m.n; t.nent = (long)ne;
+    (p->real_op ? (const void *&)t.facr : (const void *&)t.facc) = base + at[1];
+    t.outr = (double *)p->d_facr; t.outc = (double2 *)p->d_facc;
+    t.nslot = (long)p->hent.size(); t.ent = (const int2 *)(base + at[2]); t.outent = p->d_ent;
+    t.nbits = (long)m.bits.size(); t.bits = (const uint32_t *)(base + at[3]); t.outbits = p->d_bits;
+    const hipError_t e = hh::launch_operator_tables(t, c->stream);
+    if (e != hipSuccess) return fail(HH_ERR_DEVICE, "operator tables: launch failed: %s", hipGetErrorString(e));
+    HIPCHK(hipEventRecord(c->staged, c->stream));
+    if (c->stage_bytes > ((size_t)8 << 20)) {   // kept for the next operators only while it is small
+        HIPCHK(hipEventSynchronize(c->staged));
+        (void)hipHostFree(c->stage);
+        c->stage = nullptr;
+        c->stage_bytes = 0;
+    }
+    return HH_OK;
 }
 
 static int upload_plan(hh_plan *p, int ncoef, int n) {
@@ -844,17 +864,8 @@ static int upload_plan(hh_plan *p, int ncoef, int n) {
     if (rc) return rc;
     rc = dev_alloc(c, &p->coef32, b32);
     if (rc) return rc;
-    HIPCHK(hipMemcpy(p->coef64, p->hcoef.data(), b64, hipMemcpyHostToDevice));
-    std::vector<float> h32(2 * (size_t)ncoef * n * p->nop);
-    for (size_t i = 0; i < (size_t)ncoef * n * p->nop; i++) {
-        h32[2 * i] = (float)p->hcoef[i].real();
-        h32[2 * i + 1] = (float)p->hcoef[i].imag();
-    }
-    HIPCHK(hipMemcpy(p->coef32, h32.data(), b32, hipMemcpyHostToDevice));
     if ((rc = dev_alloc(c, &p->coefr64, b64 / 2))) return rc;
     if ((rc = dev_alloc(c, &p->coefr32, b32 / 2))) return rc;
-    HIPCHK(hipMemcpy(p->coefr64, p->hr64.data(), b64 / 2, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(p->coefr32, p->hr32.data(), b32 / 2, hipMemcpyHostToDevice));
     const std::vector<double> &lx = p->hlamx, &ly = p->hlamy;
     rc = dev_alloc(c, (void **)&p->lamx, lx.size() * 8);
     if (rc) return rc;
@@ -864,18 +875,13 @@ static int upload_plan(hh_plan *p, int ncoef, int n) {
         if (rc) return rc;
         HIPCHK(hipMemcpy(p->lamy, ly.data(), ly.size() * 8, hipMemcpyHostToDevice));
     }
-    if ((rc = upload_modes(p))) return rc;
+    std::lock_guard<std::mutex> lk(c->mu);
+    if ((rc = upload_tables(p))) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     return HH_OK;
 }
 
 // ------------------------------------------------------------------ host-only mode classification
-static bool table_real(const std::vector<cd> &tab) {
-    for (const cd &v : tab)
-        if (v.imag() != 0.0) return false;
-    return true;
-}
-
 extern "C" int hh_operator_modes(int dim, int Nx, int Ny, int Nz, const double *coef, double kappa, int *nflagged,
                                  int *modes, int cap, int *singular, double *kappa_worst) {
     if ((dim != 2 && dim != 3) || Nx < 2 || Ny < 2 || (dim == 3 && Nz < 2) || !coef || !(kappa >= 0) ||
@@ -911,9 +917,10 @@ extern "C" int hh_operator_mode_factors(int dim, int Nx, int Ny, int Nz, const d
     hh::ModeSet ms;
     const bool real = table_real(tab);
     hh::classify_modes(dim, Nx, Ny, Nz, 1, tab.data(), lx.data(), ly.data(), real, 0.0, ms);
-    const cd *f = ms.facc.data() + (size_t)mode * n * 4;
+    const size_t at = (size_t)mode * n * 4;
+    auto f = [&](long i) { return real ? cd(ms.facr[at + i]) : ms.facc[at + i]; };
     for (long q = 0; q < n; q++) {   // (L, R, Up) of each row
-        const cd v[3] = {f[4 * q], f[4 * q + 2], f[4 * q + 3]};
+        const cd v[3] = {f(4 * q), f(4 * q + 2), f(4 * q + 3)};
         for (int k = 0; k < 3; k++) {
             factors[2 * (3 * q + k)] = v[k].real();
             factors[2 * (3 * q + k) + 1] = v[k].imag();
@@ -1191,7 +1198,7 @@ extern "C" int hh_plan_set_resonance_threshold(hh_plan *p, double kappa) {
     hh::classify_modes(p->dim, p->Nx, p->Ny, p->Nz, p->nop, p->hcoef.data(), p->hlamx.data(), p->hlamy.data(),
                        p->real_op != 0, p->kappa_flag, p->ms);
     if (p->ms.nfx != old_nfx) p->gen++;
-    return upload_modes(p);
+    return upload_tables(p);
 }
 
 extern "C" int hh_plan_mode_info(const hh_plan *p, int op, int *flagged, int *singular, double *kappa) {
@@ -1222,8 +1229,9 @@ extern "C" int hh_plan_last_refine(const hh_plan *p, int *sweeps, double *rel) {
 // arithmetic of the tridiagonal elimination.
 // acc != 0: sol += acc A^{-1} rhs, the last pass accumulating into the FP64
 // sol (rhs is then consumed: it may serve as scratch).
+// op >= 0: the batch is one right-hand side, of operator op.
 static int solve_core(hh_plan *p, int ti, int tc, int to, int tri_comp, const void *rhs, void *sol, void *ws,
-                      int batch, double acc = 0) {
+                      int batch, double acc = 0, int op = -1) {
     hh_context *c = p->ctx;
     const int Nx = p->Nx, Ny = p->Ny, Nz = p->Nz;
     int rc;
@@ -1234,12 +1242,12 @@ static int solve_core(hh_plan *p, int ti, int tc, int to, int tri_comp, const vo
     t.coef = tri_comp == 0 ? p->coef64 : p->coef32;
     t.real = p->real_op && p->real_mode != 0;
     t.coefr = tri_comp == 0 ? p->coefr64 : p->coefr32;
-    t.nop = p->nop;
+    t.nop = op < 0 ? p->nop : 1;
     t.uni = p->d_bits;
     t.cstride = p->dim == 2 ? 6L * Ny : 12L * Nz;
     t.lamx = p->lamx; t.lamy = p->lamy;
     int n = p->dim == 2 ? Ny : Nz;
-    const long per_op = (batch + p->nop - 1) / p->nop;
+    const long per_op = (batch + t.nop - 1) / t.nop;
     builtin_tri_shape(p, tri_comp == 1, per_op, t.real, t);
     if (p->tri_W > 0 && p->tri_mm > 0) {   // shape chosen by the autotuner
         const int nr = tri_comp == 0 ? p->tri_nr : 1;
@@ -1262,6 +1270,16 @@ static int solve_core(hh_plan *p, int ti, int tc, int to, int tri_comp, const vo
         t.ent = p->d_ent;
         t.fac = t.real ? p->d_facr : p->d_facc;
         t.nent = (long)p->ms.fmode.size();
+    }
+    if (op > 0) {   // the operator's own tables; its factors are indexed through ent
+        const size_t cb = tri_comp == 0 ? 16 : 8;
+        t.coef = (const char *)t.coef + op * t.cstride * cb;
+        t.coefr = (const char *)t.coefr + op * t.cstride * (cb / 2);
+        t.uni += op;
+        if (t.nfx > 0) {
+            t.fbits += (size_t)op * t.fwords;
+            t.ent += (size_t)op * t.nfx;
+        }
     }
     auto tri = [&](void *buf) -> int {
         TimeScope ts(c, 2, (double)t.field * batch * (tc ? 16 : 32));
@@ -1428,6 +1446,22 @@ static int solve_locked(hh_plan *p, const void *rhs, void *sol, int batch) {
     size_t ws_bytes = hh_plan_workspace_bytes(p, batch);
     if (ws_bytes && (rc = ensure_scratch(c, ws_bytes))) return rc;
     return solve_ws(p, rhs, sol, batch, c->scratch);
+}
+
+// One right-hand side of a batch whose right-hand side b uses operator b, FP64:
+// the same bits as in the batch.
+int hh::solve_one(hh_plan *p, int op, const void *rhs, void *sol) {
+    if (!p || !rhs || !sol || op < 0 || op >= p->nop || p->prec != HH_PREC_F64)
+        return fail(HH_ERR_ARG, "internal: bad single solve");
+    hh_context *c = p->ctx;
+    std::lock_guard<std::mutex> lk(c->mu);
+    if (p->ms.singular[op]) return fail(HH_ERR_SINGULAR, "operator %d is singular to working precision", op);
+    int rc = set_device(c);
+    if (rc) return rc;
+    const size_t ws_bytes = hh_plan_workspace_bytes(p, 1);
+    if (ws_bytes && (rc = ensure_scratch(c, ws_bytes))) return rc;
+    void *ws = (plan_all_fft(p) && (p->dim == 3 || p->tile_w == 0)) ? nullptr : c->scratch;
+    return solve_core(p, 0, 0, 0, 0, rhs, sol, ws, 1, 0, op);
 }
 
 extern "C" int hh_solve_noalloc(hh_plan *p, const void *rhs, void *sol, int batch) {
@@ -1599,25 +1633,11 @@ extern "C" int hh_plan_set_operators(hh_plan *p, int nop, const double *coef) {
     std::lock_guard<std::mutex> lk(c->mu);
     int rc = set_device(c);
     if (rc) return rc;
-    const int nc = p->dim == 2 ? 6 : 12, n = p->dim == 2 ? p->Ny : p->Nz;
-    // the host staging buffers feed the previous call's copies until they
-    // complete; wait for the stream before refilling them
-    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));   // replaced tables may be reallocated
     const int old_real = p->real_op, old_nfx = p->ms.nfx;
     fill_table(p, nop, coef);
     if (p->real_op != old_real || p->ms.nfx != old_nfx || nop != p->nop) p->gen++;
-    if ((rc = upload_modes(p))) return rc;
-    const size_t cnt = (size_t)nc * n * nop;
-    p->h32.resize(2 * cnt);
-    for (size_t i = 0; i < cnt; i++) {
-        p->h32[2 * i] = (float)p->hcoef[i].real();
-        p->h32[2 * i + 1] = (float)p->hcoef[i].imag();
-    }
-    // stream-ordered: solves queued before this call still read the old tables
-    HIPCHK(hipMemcpyAsync(p->coef64, p->hcoef.data(), cnt * 16, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(p->coef32, p->h32.data(), cnt * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(p->coefr64, p->hr64.data(), cnt * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(p->coefr32, p->hr32.data(), cnt * 4, hipMemcpyHostToDevice, c->stream));
+    if ((rc = upload_tables(p))) return rc;   // solves queued before this call still read the old ones
     p->nop = nop;
     return HH_OK;
 }

@@ -7,6 +7,8 @@
 #include <complex>
 #include <vector>
 
+struct hh_plan;
+
 namespace hh {
 
 enum Prec { F64 = 0, F32 = 1 };
@@ -100,14 +102,35 @@ struct ModeSet {
     long nmodes = 0;
     std::vector<int> foff, fmode;         // per operator offsets (nop + 1), flagged modes
     std::vector<uint32_t> bits;           // [op] every row of its table is the same, then [op][words] flagged modes
-    std::vector<std::complex<double>> facc;   // [entry][row](L, P, R, Up)
-    std::vector<double> facr;             // real parts (real operators only)
+    std::vector<std::complex<double>> facc;   // [entry][row](L, P, R, Up), complex operators
+    std::vector<double> facr;             // the same, real operators
     std::vector<int> singular;            // per operator
     std::vector<double> kappa_worst;      // per operator: largest condition estimate of its flagged modes
 };
 // hcoef: the plan's device-order band table [op][q][6 | 12]
 void classify_modes(int dim, int Nx, int Ny, int Nz, int nop, const std::complex<double> *hcoef,
                     const double *lamx, const double *lamy, bool real, double kappa_flag, ModeSet &ms);
+
+// Sources (host-accessible or device memory) and device tables of a plan's operators.
+struct OperatorTables {
+    long ncoef = 0;                       // band table
+    const double2 *coef = nullptr;
+    double2 *coef64 = nullptr;
+    float2 *coef32 = nullptr;
+    double *coefr64 = nullptr;
+    float *coefr32 = nullptr;
+    long n = 0, nent = 0;                 // factors: rows, entries; facr where they are real, else facc
+    const double *facr = nullptr;
+    const double2 *facc = nullptr;
+    double *outr = nullptr;
+    double2 *outc = nullptr;
+    long nslot = 0, nbits = 0;            // entry slots, words of ModeSet::bits
+    const int2 *ent = nullptr;
+    int2 *outent = nullptr;
+    const uint32_t *bits = nullptr;
+    uint32_t *outbits = nullptr;
+};
+hipError_t launch_operator_tables(const OperatorTables &t, hipStream_t st);
 
 // Choose a tridiagonal block shape for a system of length n and nmodes modes.
 void tri_shape(int n, long nmodes, int *W, int *P, int *mmax);
@@ -168,5 +191,8 @@ hipError_t launch_residual_norms(void *norms, double *out, hipStream_t st);
 constexpr int NORM_BLOCKS = 2048;
 hipError_t launch_norms(long n, const void *x, const void *y, double *part, double *out, hipStream_t st,
                         bool l2 = false);
+
+// For the serving loop (hh_api.hip): right-hand side and operator `op` of a plan alone.
+int solve_one(hh_plan *p, int op, const void *rhs, void *sol);
 
 }  // namespace hh

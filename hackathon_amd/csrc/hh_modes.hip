@@ -35,6 +35,7 @@
 // operator singular to working precision: the plan reports HH_ERR_SINGULAR
 // for solves that use it.  The reference divides by such pivots unchecked
 // (2D LU.c:36, 3D LU.c:68).
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstdint>
@@ -76,54 +77,62 @@ inline RowBands row_bands(int dim, const cd *row, double lx, double ly, double l
     return r;
 }
 
-// Real-operator factors, reference order, FP64 with no fused operations.
+// Real-operator factors of G modes, reference order, FP64 with no fused operations.
 // out rows: (L_q, P_q, R_q, Up_q).  2D: the reference divides by its pivot
 // U_q; P_q = U_q and R_q = RN(1/U_q), with which the device reproduces the
 // correctly rounded quotient (one fused correction step, Markstein).  3D:
 // the reference multiplies by its stored reciprocal pivot U_q; R_q = U_q and
-// P_q = 1/U_q (unused).  Returns false when a pivot is zero or not finite.
-bool factors_real(int dim, int n, const cd *tab, int nc, double lx, double ly, double lxy, double *out) {
-    bool ok = true;
-    double Uprev = 0, Upprev = 0;
+// P_q = 1/U_q (unused).  ok: no pivot is zero or not finite.
+// Each mode is a serial chain of divisions; G of them side by side keep the
+// divider busy, and one mode's operations do not change (1023 rows, 11 modes
+// with their condition estimates: 309 us one by one, 92 in groups of 4, on the
+// host while a serving loop's GPU waits).
+constexpr int GROUP = 4;
+template <int DIM>
+void factors_real(int n, const cd *tab, const double *lx, const double *ly, double *const *out, bool *ok) {
+    constexpr int NC = DIM == 2 ? 6 : 12;
+    double Uprev[GROUP] = {}, Upprev[GROUP] = {}, bad[GROUP] = {}, lxy[GROUP];
+    for (int g = 0; g < GROUP; g++) lxy[g] = lx[g] * ly[g];
     for (int q = 0; q < n; q++) {
-        const cd *row = tab + (long)q * nc;
-        double sub, dia, sup;
-        if (dim == 2) {
-            sub = row[0].real() * lx + row[1].real();
-            dia = row[2].real() * lx + row[3].real();
-            sup = row[4].real() * lx + row[5].real();
-        } else {
-            auto e = [&](const cd *c) {
-                return ((c[0].real() * lxy + c[1].real() * lx) + c[2].real() * ly) + c[3].real();
-            };
-            dia = e(row);
-            sup = e(row + 4);
-            sub = e(row + 8);
+        const cd *row = tab + (long)q * NC;
+        double L[GROUP], U[GROUP], R[GROUP], P[GROUP], sup[GROUP];
+        for (int g = 0; g < GROUP; g++) {
+            double sub, dia;
+            if constexpr (DIM == 2) {
+                sub = row[0].real() * lx[g] + row[1].real();
+                dia = row[2].real() * lx[g] + row[3].real();
+                sup[g] = row[4].real() * lx[g] + row[5].real();
+                // LU.c:32-40: L = sub / U_{q-1}, U = dia - L Up_{q-1}
+                L[g] = q == 0 ? 0.0 : sub / Uprev[g];
+                U[g] = q == 0 ? dia : dia - L[g] * Upprev[g];
+                R[g] = 1.0 / U[g];
+                P[g] = U[g];
+            } else {
+                auto e = [&](const cd *c) {
+                    return ((c[0].real() * lxy[g] + c[1].real() * lx[g]) + c[2].real() * ly[g]) + c[3].real();
+                };
+                dia = e(row);
+                sup[g] = e(row + 4);
+                sub = e(row + 8);
+                // LU.c:61-72: L = sub U_{q-1} (U reciprocal), U = 1 / (dia - Up_{q-1} L)
+                L[g] = q == 0 ? 0.0 : sub * Uprev[g];
+                U[g] = q == 0 ? 1.0 / dia : 1.0 / (dia - Upprev[g] * L[g]);
+                R[g] = U[g];
+                P[g] = 1.0 / U[g];
+            }
+            bad[g] += (L[g] - L[g]) + (R[g] - R[g]) + (P[g] - P[g]);   // zero, or NaN once a value is not finite
+            Uprev[g] = U[g];
+            Upprev[g] = sup[g];
         }
-        double L, U, R, P;
-        if (dim == 2) {
-            // LU.c:32-40: L = sub / U_{q-1}, U = dia - L Up_{q-1}
-            L = q == 0 ? 0.0 : sub / Uprev;
-            U = q == 0 ? dia : dia - L * Upprev;
-            R = 1.0 / U;
-            P = U;
-            Uprev = U;
-        } else {
-            // LU.c:61-72: L = sub U_{q-1} (U reciprocal), U = 1 / (dia - Up_{q-1} L)
-            L = q == 0 ? 0.0 : sub * Uprev;
-            U = q == 0 ? 1.0 / dia : 1.0 / (dia - Upprev * L);
-            R = U;
-            P = 1.0 / U;
-            Uprev = U;
+        for (int g = 0; g < GROUP; g++) {
+            double *o = out[g] + 4 * (long)q;
+            o[0] = L[g];
+            o[1] = P[g];
+            o[2] = R[g];
+            o[3] = q == n - 1 ? 0.0 : sup[g];   // the last row has no superdiagonal
         }
-        if (!std::isfinite(L) || !std::isfinite(R) || !std::isfinite(P) || U == 0.0) ok = false;
-        Upprev = sup;
-        out[4 * q] = L;
-        out[4 * q + 1] = P;
-        out[4 * q + 2] = R;
-        out[4 * q + 3] = q == n - 1 ? 0.0 : sup;   // the last row has no superdiagonal
     }
-    return ok;
+    for (int g = 0; g < GROUP; g++) ok[g] = bad[g] == 0.0;
 }
 
 bool factors_complex(int dim, int n, const cd *tab, int nc, double lx, double ly, double lxy, cd *out) {
@@ -155,27 +164,80 @@ bool factors_complex(int dim, int n, const cd *tab, int nc, double lx, double ly
 }
 #pragma clang fp contract(on)
 
-// ||T^{-1} e||_inf for e = all ones and e = a fixed +-1 pattern, with the
-// factors (L, P, R, Up) of the reference substitution.
-template <typename V> double inv_norm_est(int n, const V *f) {
-    double best = 0;
-    std::vector<V> y(n);
-    for (int pass = 0; pass < 2; pass++) {
-        uint32_t s = 0x9e3779b9u;
-        for (int q = 0; q < n; q++) {
-            double e = 1.0;
-            if (pass) { s = s * 1664525u + 1013904223u; e = (s >> 31) ? 1.0 : -1.0; }
-            y[q] = q == 0 ? V(e) : V(e) - f[4 * q] * y[q - 1];
+// Varah margin min (|dia| - |sub| - |sup|) and row sum max (|dia| + |sub| +
+// |sup|) of G modes over rows qbeg .. qend - 1.  Magnitudes as sqrt(re^2 +
+// im^2): the bands are far from overflow, std::abs's hypot costs several times more.
+template <int DIM, bool REAL>
+void mode_bounds(int n, const cd *tab, int qbeg, int qend, const double *lx, const double *ly, double *margin,
+                 double *rowsum) {
+    constexpr int NC = DIM == 2 ? 6 : 12;
+    double mn[GROUP], mx[GROUP], lxy[GROUP];
+    for (int g = 0; g < GROUP; g++) { mn[g] = INFINITY; mx[g] = 0; lxy[g] = lx[g] * ly[g]; }
+    for (int q = qbeg; q < qend; q++) {
+        const cd *c = tab + (long)q * NC;
+        double s[GROUP], d[GROUP], u[GROUP];
+        auto part = [&](auto at, double *out) {   // |band| of the coefficients at(i), componentwise
+            double re[GROUP], im[GROUP];
+            for (int g = 0; g < GROUP; g++) {
+                if constexpr (DIM == 2) {
+                    re[g] = at(0).real() * lx[g] + at(1).real();
+                    im[g] = REAL ? 0.0 : at(0).imag() * lx[g] + at(1).imag();
+                } else {
+                    re[g] = at(0).real() * lxy[g] + at(1).real() * lx[g] + at(2).real() * ly[g] + at(3).real();
+                    im[g] = REAL ? 0.0 : at(0).imag() * lxy[g] + at(1).imag() * lx[g] + at(2).imag() * ly[g] + at(3).imag();
+                }
+            }
+            for (int g = 0; g < GROUP; g++)
+                out[g] = REAL ? std::fabs(re[g]) : __builtin_sqrt(re[g] * re[g] + im[g] * im[g]);
+        };
+        if constexpr (DIM == 2) {   // (bm, am, b, a, bp, ap)
+            part([&](int i) { return c[i]; }, s);
+            part([&](int i) { return c[2 + i]; }, d);
+            part([&](int i) { return c[4 + i]; }, u);
+        } else {   // (a..d, ap..dp, am..dm)
+            part([&](int i) { return c[i]; }, d);
+            part([&](int i) { return c[4 + i]; }, u);
+            part([&](int i) { return c[8 + i]; }, s);
         }
-        V x = 0;
-        double mx = 0;
-        for (int q = n - 1; q >= 0; q--) {
-            x = q == n - 1 ? y[q] * f[4 * q + 2] : (y[q] - f[4 * q + 3] * x) * f[4 * q + 2];
-            mx = std::max(mx, std::abs(x));
+        for (int g = 0; g < GROUP; g++) {
+            const double sg = q == 0 ? 0.0 : s[g], ug = q == n - 1 ? 0.0 : u[g];
+            const double a = d[g] - sg - ug, b = d[g] + sg + ug;
+            mn[g] = a < mn[g] ? a : mn[g];
+            mx[g] = mx[g] < b ? b : mx[g];
         }
-        best = std::max(best, mx);
     }
-    return best;
+    for (int g = 0; g < GROUP; g++) { margin[g] = mn[g]; rowsum[g] = mx[g]; }
+}
+
+// ||T^{-1} e||_inf for e = all ones and e = a fixed +-1 pattern, with the
+// factors (L, P, R, Up) of the reference substitution, for G systems; y: 2 n G values.
+template <typename V, int G> void inv_norm_est(int n, const V *const *f, std::vector<V> &y, double *inv) {
+    y.resize(2 * (size_t)n * G);
+    V last[2 * G] = {};
+    uint32_t s = 0x9e3779b9u;
+    for (int q = 0; q < n; q++) {
+        s = s * 1664525u + 1013904223u;
+        const double e[2] = {1.0, (s >> 31) ? 1.0 : -1.0};
+        V *yq = y.data() + 2 * (size_t)G * q;
+        for (int g = 0; g < G; g++) {
+            const V L = f[g][4 * (long)q];
+            for (int k = 0; k < 2; k++) yq[2 * g + k] = last[2 * g + k] = q == 0 ? V(e[k]) : V(e[k]) - L * last[2 * g + k];
+        }
+    }
+    V x[2 * G] = {};
+    double mx[2 * G] = {};
+    for (int q = n - 1; q >= 0; q--) {
+        const V *yq = y.data() + 2 * (size_t)G * q;
+        for (int g = 0; g < G; g++) {
+            const V R = f[g][4 * (long)q + 2], up = f[g][4 * (long)q + 3];
+            for (int k = 0; k < 2; k++) {
+                const int i = 2 * g + k;
+                x[i] = q == n - 1 ? yq[i] * R : (yq[i] - up * x[i]) * R;
+                mx[i] = std::max(mx[i], std::abs(x[i]));
+            }
+        }
+    }
+    for (int g = 0; g < G; g++) inv[g] = std::max(std::max(0.0, mx[2 * g]), mx[2 * g + 1]);
 }
 
 }  // namespace
@@ -197,7 +259,8 @@ void classify_modes(int dim, int Nx, int Ny, int Nz, int nop, const cd *hcoef, c
     ms.singular.assign(nop, 0);
     ms.kappa_worst.assign(nop, 0.0);
     ms.nfx = 0;
-    std::vector<RowBands> rows(n);
+    std::vector<double> yr, sums;
+    std::vector<cd> yc;
     for (int o = 0; o < nop; o++) {
         const cd *tab = hcoef + (size_t)o * n * nc;
         // a table whose rows are all equal (constant k) gives every interior
@@ -208,70 +271,102 @@ void classify_modes(int dim, int Nx, int Ny, int Nz, int nop, const cd *hcoef, c
                 if (tab[(long)q * nc + t] != tab[t]) { uniform = false; break; }
         ms.bits[o] = uniform;
         ms.foff[o] = (int)ms.fmode.size();
+        // equal rows: an inner one has the smallest margin and the largest sum
+        const int qbeg = uniform && n > 2 ? 1 : 0, qend = uniform ? std::min(n, 2) : n;
+        auto bounds = dim == 2 ? (real ? mode_bounds<2, true> : mode_bounds<2, false>)
+                               : (real ? mode_bounds<3, true> : mode_bounds<3, false>);
+        double margins[GROUP], rowsums[GROUP];
         for (long m = 0; m < nmodes; m++) {
-            const double lx = dim == 2 ? lamx[m] : lamx[m % Nx];
-            const double ly = dim == 2 ? 0.0 : lamy[m / Nx];
-            const double lxy = lx * ly;
-            double margin = INFINITY, rowsum = 0;
-            const int qend = uniform ? std::min(n, 3) : n;
-            for (int q = 0; q < qend; q++) {
-                // magnitudes as sqrt(re^2 + im^2) (the bands are far from
-                // overflow; std::abs's hypot costs several times more, and a
-                // serving loop classifies every request's operator)
-                double s, d, u;
-                if (real) {
-                    const cd *row = tab + (long)q * nc;
-                    double sub, dia, sup;
-                    if (dim == 2) {
-                        sub = row[0].real() * lx + row[1].real();
-                        dia = row[2].real() * lx + row[3].real();
-                        sup = row[4].real() * lx + row[5].real();
-                    } else {
-                        auto e = [&](const cd *c) {
-                            return c[0].real() * lxy + c[1].real() * lx + c[2].real() * ly + c[3].real();
-                        };
-                        dia = e(row);
-                        sup = e(row + 4);
-                        sub = e(row + 8);
-                    }
-                    s = std::fabs(sub); d = std::fabs(dia); u = std::fabs(sup);
-                } else {
-                    const RowBands b = row_bands(dim, tab + (long)q * nc, lx, ly, lxy);
-                    auto mag = [](cd z) { return std::sqrt(z.real() * z.real() + z.imag() * z.imag()); };
-                    s = mag(b.sub); d = mag(b.dia); u = mag(b.sup);
+            const int g = (int)(m % GROUP);
+            if (g == 0) {
+                double lx[GROUP], ly[GROUP];
+                for (int i = 0; i < GROUP; i++) {
+                    const long mm = std::min(m + i, nmodes - 1);
+                    lx[i] = dim == 2 ? lamx[mm] : lamx[mm % Nx];
+                    ly[i] = dim == 2 ? 0.0 : lamy[mm / Nx];
                 }
-                if (q == 0) s = 0.0;
-                if (q == n - 1) u = 0.0;
-                margin = std::min(margin, d - s - u);
-                rowsum = std::max(rowsum, d + s + u);
+                bounds(n, tab, qbeg, qend, lx, ly, margins, rowsums);
             }
+            const double margin = margins[g], rowsum = rowsums[g];
             const bool flag = !(margin > 0) || rowsum > kappa_flag * margin;
             if (!flag) continue;
-            const long e = (long)ms.fmode.size();
             ms.fmode.push_back((int)m);
             ms.bits[nop + (size_t)o * ms.words + m / 32] |= 1u << (m % 32);
-            ms.facc.resize((size_t)(e + 1) * n * 4);
-            cd *fc = ms.facc.data() + (size_t)e * n * 4;
-            bool ok;
-            double inv;
-            if (real) {
-                std::vector<double> fr(4 * (size_t)n);
-                ok = factors_real(dim, n, tab, nc, lx, ly, lxy, fr.data());
-                for (size_t i = 0; i < fr.size(); i++) fc[i] = fr[i];
-                ms.facr.insert(ms.facr.end(), fr.begin(), fr.end());
-                inv = ok ? inv_norm_est<double>(n, fr.data()) : INFINITY;
-            } else {
-                ok = factors_complex(dim, n, tab, nc, lx, ly, lxy, fc);
-                inv = ok ? inv_norm_est<cd>(n, fc) : INFINITY;
+            sums.push_back(rowsum);
+        }
+        // factors and condition estimates of the operator's flagged modes
+        const size_t e0 = ms.foff[o], e1 = ms.fmode.size(), len = 4 * (size_t)n;
+        if (real) ms.facr.resize(e1 * len);
+        else ms.facc.resize(e1 * len);
+        for (size_t e = e0; e < e1; e += real ? GROUP : 1) {
+            bool ok[GROUP];
+            double lx[GROUP], ly[GROUP], inv[GROUP];
+            const int ng = real ? (int)std::min<size_t>(GROUP, e1 - e) : 1;
+            for (int g = 0; g < GROUP; g++) {   // a last group repeats its last mode
+                const long m = ms.fmode[e + std::min(g, ng - 1)];
+                lx[g] = dim == 2 ? lamx[m] : lamx[m % Nx];
+                ly[g] = dim == 2 ? 0.0 : lamy[m / Nx];
             }
-            const double kap = rowsum * inv;
-            if (!ok || !std::isfinite(kap) || kap > HH_SINGULAR_KAPPA) ms.singular[o] = 1;
-            if (!(kap <= ms.kappa_worst[o])) ms.kappa_worst[o] = kap;
+            if (real) {
+                double *out[GROUP];
+                for (int g = 0; g < GROUP; g++) out[g] = ms.facr.data() + (e + std::min(g, ng - 1)) * len;
+                if (dim == 2) factors_real<2>(n, tab, lx, ly, out, ok);
+                else factors_real<3>(n, tab, lx, ly, out, ok);
+                inv_norm_est<double, GROUP>(n, out, yr, inv);
+            } else {
+                cd *out = ms.facc.data() + e * len;
+                ok[0] = factors_complex(dim, n, tab, nc, lx[0], ly[0], lx[0] * ly[0], out);
+                inv_norm_est<cd, 1>(n, &out, yc, inv);
+            }
+            for (int g = 0; g < ng; g++) {
+                const double kap = sums[e + g] * (ok[g] ? inv[g] : INFINITY);
+                if (!ok[g] || !std::isfinite(kap) || kap > HH_SINGULAR_KAPPA) ms.singular[o] = 1;
+                if (!(kap <= ms.kappa_worst[o])) ms.kappa_worst[o] = kap;
+            }
         }
         const int cnt = (int)ms.fmode.size() - ms.foff[o];
         if (cnt > ms.nfx) ms.nfx = cnt;
     }
     ms.foff[nop] = (int)ms.fmode.size();
+}
+
+// Device tables of a plan's operators from their host form: one launch for
+// what took up to eight copies of pageable memory (a serving loop's batch of
+// three 1023-row operators: 150 us of copies that queued behind its
+// right-hand sides on the copy engine).  The sources are read once, over the
+// link when they are in host memory; the FP32 and real forms of the bands,
+// the complex form of real factors and the factors' device order
+// [row][entry](L, P, R, Up), in which the lanes of neighbouring entries read
+// neighbouring records, are made here and do not cross it.
+__global__ __launch_bounds__(256) void k_operator_tables(OperatorTables t) {
+    const long id = (long)blockIdx.x * 256 + threadIdx.x, step = (long)gridDim.x * 256;
+    for (long i = id; i < t.ncoef; i += step) {
+        const double2 v = t.coef[i];
+        t.coef64[i] = v;
+        t.coef32[i] = make_float2((float)v.x, (float)v.y);
+        t.coefr64[i] = v.x;
+        t.coefr32[i] = (float)v.x;
+    }
+    const long per = 4L * t.n;   // values of one entry
+    for (long i = id; i < t.nent * per; i += step) {
+        const long e = i / per, r = i - e * per, q = r >> 2, to = (q * t.nent + e) * 4 + (r & 3);
+        if (t.facr) {
+            const double v = t.facr[i];
+            t.outr[to] = v;
+            t.outc[to] = make_double2(v, 0.0);
+        } else {
+            t.outc[to] = t.facc[i];
+        }
+    }
+    for (long i = id; i < t.nslot; i += step) t.outent[i] = t.ent[i];
+    for (long i = id; i < t.nbits; i += step) t.outbits[i] = t.bits[i];
+}
+
+hipError_t launch_operator_tables(const OperatorTables &t, hipStream_t st) {
+    const long work = std::max(std::max(t.ncoef, 4 * t.nent * t.n), std::max(t.nslot, t.nbits));
+    const long blocks = std::min(1024L, (work + 255) / 256);
+    hipLaunchKernelGGL(k_operator_tables, dim3((unsigned)std::max(1L, blocks)), dim3(256), 0, st, t);
+    return hipGetLastError();
 }
 
 }  // namespace hh
