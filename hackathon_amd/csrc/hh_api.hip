@@ -1318,20 +1318,24 @@ static int solve_core(hh_plan *p, int ti, int tc, int to, int tri_comp, const vo
     if (acc != 0 && (to != 0 || ti != tc)) return fail(HH_ERR_UNSUPPORTED, "internal: accumulating solve types");
     hh::Lines lx = rows_lines(Nx, (long)Ny * Nz * batch);
     hh::Lines ly = cols_lines(Nx, Ny, (long)Nz * batch);
+    // FFT passes start where the pass before ended: y backwards before the mode
+    // solves, x after them (255^3: 525 -> 514 us; smaller fields fit the cache either way)
+    hh::Lines lyr = ly, lxr = lx;
+    lyr.reverse = lxr.reverse = 1;
     if (fft && tc == to && acc == 0) {
         if ((rc = dst_pass(c, lx, ti, tc, tc, rhs, sol))) return rc;
-        if ((rc = dst_pass(c, ly, tc, tc, tc, sol, sol))) return rc;
+        if ((rc = dst_pass(c, lyr, tc, tc, tc, sol, sol))) return rc;
         if ((rc = tri(sol))) return rc;
         if ((rc = dst_pass(c, ly, tc, tc, tc, sol, sol))) return rc;
-        return dst_pass(c, lx, tc, tc, to, sol, sol);
+        return dst_pass(c, lxr, tc, tc, to, sol, sol);
     }
     if (!ws) return fail(HH_ERR_ARG, "internal: missing workspace");
     if (fft) {   // intermediate precision differs from the output: keep it in ws
         if ((rc = dst_pass(c, lx, ti, tc, tc, rhs, ws))) return rc;
-        if ((rc = dst_pass(c, ly, tc, tc, tc, ws, ws))) return rc;
+        if ((rc = dst_pass(c, lyr, tc, tc, tc, ws, ws))) return rc;
         if ((rc = tri(ws))) return rc;
         if ((rc = dst_pass(c, ly, tc, tc, tc, ws, ws))) return rc;
-        return dst_pass(c, lx, tc, tc, to, ws, sol, acc);
+        return dst_pass(c, lxr, tc, tc, to, ws, sol, acc);
     }
     // dense 3D path: ping-pong between ws and a second buffer holding the
     // intermediate in the compute type: sol (no smaller than the compute

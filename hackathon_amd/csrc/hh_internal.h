@@ -42,6 +42,9 @@ struct Lines {
     // (FP64) output instead of storing it, out += acc X (the update of an
     // iterative refinement applied as the last pass stores).
     double acc = 0;
+    // Blocks take the last lines first: the pass before wrote those last, so
+    // they are the ones still in the memory-side cache.
+    int reverse = 0;
 };
 
 // Tables of the dense DST: two matrices (odd outputs, then even ones) of

@@ -44,6 +44,18 @@ def test_columns(Nx, Ny, layers):
     assert torch.equal(torch.view_as_real(a), torch.view_as_real(b))
 
 
+# planes are dealt to the XCDs eight at a time, the rest in order
+@pytest.mark.parametrize("Nx,Ny", [(63, 15), (255, 127), (300, 31)])
+@pytest.mark.parametrize("layers", [1, 7, 8, 9, 16, 23])
+def test_layers_alone(Nx, Ny, layers):
+    from hackathon_amd import helmholtz as H
+    ctx = H.Context(0)
+    x = noise(layers, Ny, Nx)
+    got = ctx.dst2d_layers(x)
+    want = torch.stack([ctx.dst2d_layers(x[i:i + 1].contiguous())[0] for i in range(layers)])
+    assert torch.equal(torch.view_as_real(got), torch.view_as_real(want))
+
+
 # FP32 spectra of a mixed-precision solve, around the edges of its row (128 and
 # 192 blocks at N + 1 = 256) and wide-tile rules (448 and 1024 blocks at 128)
 @pytest.mark.parametrize("dims", [(255, 100, 1), (255, 192 * 16, 1), (255, 193 * 16, 1), (31, 31, 20), (63, 63, 128),
