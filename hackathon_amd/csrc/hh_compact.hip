@@ -20,9 +20,11 @@
 //
 // What bounds it: memory, 5 (2D) and 10 (3D) fields moved, where derivative
 // fields on the extended grid, their zeroing and a separate combination took
-// 14 and 24.  8 x 1023^2: x 78 us (3.5 TB/s), y 150 us (2.7 TB/s: 128-byte
-// segments 16 KB apart), before 478 us in five kernels; 200^3: x 78, y 125, z 112
+// 14 and 24.  8 x 1023^2: x 75 us (3.6 TB/s), y 150 us (2.7 TB/s: 128-byte
+// segments 16 KB apart), before 478 us in five kernels; 200^3: x 65, y 125, z 112
 // us (4.6 TB/s), before 615 us in six.
+#include <algorithm>
+
 #include "hh_closure.h"
 #include "hh_common.h"
 #include "hh_internal.h"
@@ -44,11 +46,19 @@ HH_DEV z2 zf(z2 a, double s, z2 b) { return mk<double>(__builtin_fma(s, b.x, a.x
 
 // Thread (w, c) of a block holds rows c MM .. c MM + MM - 1 of line w.  The
 // reciprocal pivots R_0 = 1/diag, R_q = 1/(diag - R_{q-1}) reach their limit
-// to the last bit within 16 rows for both diagonals.
+// to the last bit within 16 rows for both diagonals; they are constants (17
+// divisions, one after the other, kept each block's first loads waiting).
 constexpr int CPIV = 16;
-HH_DEV void pivot_table(double diag, double *R) {   // CPIV + 1 values, by one thread
+struct Pivots { double r[CPIV + 1]; };
+constexpr Pivots pivots(double diag) {
+    Pivots p{};
     double r = 1.0 / diag;
-    for (int q = 0; q <= CPIV; q++) { R[q] = r; r = 1.0 / (diag - r); }
+    for (int q = 0; q <= CPIV; q++) { p.r[q] = r; r = 1.0 / (diag - r); }
+    return p;
+}
+__constant__ const Pivots PIVOTS[2] = {pivots(10.0), pivots(4.0)};
+template <int DIAG> HH_DEV void pivot_table(double *R) {
+    if (threadIdx.x <= CPIV) R[threadIdx.x] = PIVOTS[DIAG == 4].r[threadIdx.x];
 }
 HH_DEV double pivot(const double *R, int q) { return R[q < CPIV ? q : CPIV]; }
 
@@ -145,7 +155,8 @@ HH_DEV long xcd_order(long b, long G) {
 // nA) + (l / nA) eA.
 struct XLines {
     int n, W, P;
-    long nlines, nA, fB, fO, fC, oB, eB, e0, eA;
+    int nlines, nA;
+    long fB, fO, fC, oB, eB, e0, eA;
     const z2 *f, *lo, *hi;
     z2 *out;
     double rh2;   // 12 / h^2
@@ -159,44 +170,49 @@ constexpr int line_pad(int i) { return i + (i >> 3); }
 template <int MM, bool STAGE>
 __global__ __launch_bounds__(1024) void k_compact_x(XLines a, int b0) {
     extern __shared__ __align__(16) unsigned char smem[];
-    const int n = a.n, P = a.P, W = a.W, NT = blockDim.x;
+    const int n = a.n, P = a.P, W = a.W, nt = blockDim.x;
     Exchange ex(smem, P, W);
     z2 *line = reinterpret_cast<z2 *>(smem + (Exchange::bytes(P, W) + 15) / 16 * 16);
     const int LS = line_pad(n + 2) + 1;
     const int t = threadIdx.x;
     const int b = b0 + blockIdx.y;
-    const long l0 = (long)blockIdx.x * W;
-    const int nl = (int)(a.nlines - l0 < W ? a.nlines - l0 : W);
-    auto fbase = [&](long l) { return b * a.fB + (l / a.nA) * a.fO + (l % a.nA + 1) * (long)(n + 2) + a.fC; };
-    if (t == 0) pivot_table(10.0, ex.R);
+    const int l0 = blockIdx.x * W;
+    const int nl = min(a.nlines - l0, W);
+    // this thread's line: its first ghost in f and its boundary values, asked for first
+    const int w = min(t / P, W - 1), c = t - w * P;
+    const bool live = c < P && w < nl;
+    const int q0 = live ? c * MM : 0;
+    const int l = l0 + (live ? w : 0), outer = (unsigned)l / (unsigned)a.nA, inner = l - outer * a.nA;
+    const long fbase = b * a.fB + outer * a.fO + (inner + 1) * (long)(n + 2) + a.fC;
+    const long eo = b * a.eB + a.e0 + inner + outer * a.eA;
+    const z2 lo = a.lo[eo], hi = a.hi[eo];
+    pivot_table<10>(ex.R);
     if constexpr (STAGE) {
-        long *base = reinterpret_cast<long *>(ex.ye);   // one 64-bit division per line, not per element
-        if (t < nl) base[t] = fbase(l0 + t);
+        long *base = reinterpret_cast<long *>(ex.ye);
+        if (live && c == 0) base[w] = fbase;
         __syncthreads();
         const int total = nl * (n + 2);   // eight loads in flight per thread
-        for (int e0 = t; e0 < total; e0 += 8 * NT) {
+        // e / (n + 2) by a reciprocal, exact below 2^21 elements (the tile fits the LDS)
+        const float inv = 1.0f / (float)(n + 2);
+        for (int e0 = t; e0 < total; e0 += 8 * nt) {
             z2 g[8];
             int pos[8];
 #pragma unroll
             for (int k = 0; k < 8; k++) {
-                const int e = min(e0 + k * NT, total - 1), w = e / (n + 2), i = e - w * (n + 2);
+                const int e = min(e0 + k * nt, total - 1), w = (int)(((float)e + 0.5f) * inv), i = e - w * (n + 2);
                 pos[k] = w * LS + line_pad(i);
                 g[k] = a.f[base[w] + i];
             }
 #pragma unroll
             for (int k = 0; k < 8; k++)
-                if (e0 + k * NT < total) line[pos[k]] = g[k];
+                if (e0 + k * nt < total) line[pos[k]] = g[k];
         }
     }
     __syncthreads();
-    const int w = min(t / P, W - 1), c = t - w * P;
-    const bool live = c < P && w < nl;
-    const int q0 = live ? c * MM : 0;
-    const long l = l0 + (live ? w : 0);
     z2 v[MM];
     {
         z2 g[MM + 2];
-        const long src = STAGE ? (live ? w : 0) * LS : fbase(l);
+        const long src = STAGE ? (live ? w : 0) * LS : fbase;
 #pragma unroll
         for (int k = 0; k < MM + 2; k++) {
             const int i = min(q0 + k, n + 1);
@@ -207,9 +223,8 @@ __global__ __launch_bounds__(1024) void k_compact_x(XLines a, int b0) {
         for (int k = 0; k < MM; k++) {
             v[k] = zsel(q0 + k < n, zs(za(zd(g[k], zs(g[k + 1], 2.0)), g[k + 2]), a.rh2));
         }
-        const long eo = b * a.eB + a.e0 + l % a.nA + (l / a.nA) * a.eA;
-        if (q0 == 0) v[0] = zd(v[0], a.lo[eo]);
-        if (q0 + MM >= n) subtract_last<MM>(v, n - 1 - q0, a.hi[eo]);
+        if (q0 == 0) v[0] = zd(v[0], lo);
+        if (q0 + MM >= n) subtract_last<MM>(v, n - 1 - q0, hi);
     }
     constexpr int LV = Levels<MM, 10>::LV;
     z2 end;
@@ -234,7 +249,7 @@ __global__ __launch_bounds__(1024) void k_compact_x(XLines a, int b0) {
         __syncthreads();
         z2 *dst = a.out + b * a.oB + l0 * (long)n;
         for (int w2 = 0; w2 < nl; w2++)
-            for (int i = t; i < n; i += NT) dst[(long)w2 * n + i] = line[w2 * LS + line_pad(i)];
+            for (int i = t; i < n; i += nt) dst[(long)w2 * n + i] = line[w2 * LS + line_pad(i)];
     }
 }
 
@@ -279,8 +294,8 @@ template <int MM, bool FY> __global__ __launch_bounds__(FY ? 512 : 1024) void k_
     extern __shared__ __align__(16) unsigned char smem[];
     const int n = a.s.n, P = a.s.P, W = a.s.W, Nx = a.s.Nx, X = Nx + 2;
     Exchange e2(smem, P, W), e1(smem + (Exchange::bytes(P, W) + 15) / 16 * 16, P, W);
-    if (threadIdx.x == 0) pivot_table(10.0, e2.R);
-    if (FY && threadIdx.x == 1) pivot_table(4.0, e1.R);
+    pivot_table<10>(e2.R);
+    if constexpr (FY) pivot_table<4>(e1.R);
     int w, c, i;
     bool live;
     strided_thread(a.s, w, c, i, live);
@@ -384,7 +399,7 @@ template <int MM> __global__ __launch_bounds__(1024) void k_rhs3d_6y(Y3D a, int 
     extern __shared__ __align__(16) unsigned char smem[];
     const int n = a.s.n, P = a.s.P, W = a.s.W, Nx = a.s.Nx;
     Exchange ex(smem, P, W);
-    if (threadIdx.x == 0) pivot_table(10.0, ex.R);
+    pivot_table<10>(ex.R);
     int w, c, i;
     bool live;
     strided_thread(a.s, w, c, i, live);
@@ -461,7 +476,7 @@ template <int MM> __global__ __launch_bounds__(1024) void k_rhs3d_6z(Z3D a, int 
     extern __shared__ __align__(16) unsigned char smem[];
     const int n = a.s.n, P = a.s.P, W = a.s.W, Nx = a.NX, Ny = a.NY;
     Exchange ex(smem, P, W);
-    if (threadIdx.x == 0) pivot_table(10.0, ex.R);
+    pivot_table<10>(ex.R);
     int w, c, m;
     bool live;
     strided_thread(a.s, w, c, m, live);
@@ -546,22 +561,22 @@ template <class K> hipError_t with_lds(K kfn, size_t shm) {
 }
 
 hipError_t launch_x(XLines a, int batch, hipStream_t st) {
+    const size_t per_line = (size_t)(line_pad(a.n + 2) + 1) * 16;
+    auto lds = [&](int P, int W) { return (Exchange::bytes(P, W) + 15) / 16 * 16 + W * per_line; };
     const int mm = chunk_rows(a.n);
     a.P = (a.n + mm - 1) / mm;
     if (a.P > 1024) return hipErrorInvalidValue;
-    const size_t per_line = (size_t)(line_pad(a.n + 2) + 1) * 16;
-    const size_t room = 160 * 1024 - 1024;
-    // about 256 threads per block (77 us at 8 x 1023^2, 80 with 512)
-    a.W = 256 / a.P > 0 ? 256 / a.P : 1;
-    if ((long)a.W > a.nlines) a.W = (int)a.nlines;
-    auto lds = [&](int W) { return (Exchange::bytes(a.P, W) + 15) / 16 * 16 + W * per_line; };
-    const bool stage = mm == 8 && lds(1) <= room;
-    while (stage && a.W > 1 && lds(a.W) > room / 2) a.W--;
-    const size_t shm = stage ? lds(a.W) : Exchange::bytes(a.P, a.W);
+    const bool stage = mm == 8 && lds(a.P, 1) <= 160 * 1024 - 1024;
+    // one wave per block where lines are short: its barriers wait for no other
+    // (200^3: 65 us, 74 with 256 threads; 8 x 1023^2, 128 threads a line: 75 and 74;
+    // 16 rows per thread, one wave a line there: 100)
+    a.W = std::max(1, 64 / a.P);
+    if (a.W > a.nlines) a.W = a.nlines;
+    const size_t shm = stage ? lds(a.P, a.W) : Exchange::bytes(a.P, a.W);
     auto kfn = !stage ? (mm == 8 ? k_compact_x<8, false> : k_compact_x<16, false>) : k_compact_x<8, true>;
     hipError_t e = with_lds(kfn, shm);
     if (e != hipSuccess) return e;
-    const long tiles = (a.nlines + a.W - 1) / a.W;
+    const long tiles = ((long)a.nlines + a.W - 1) / a.W;
     const int threads = (a.W * a.P + 63) / 64 * 64;
     for (int b0 = 0; b0 < batch; b0 += 65535) {
         const int nb = batch - b0 < 65535 ? batch - b0 : 65535;
@@ -608,7 +623,8 @@ hipError_t launch_rhs3d_6(const Rhs3D &r, void *F, hipStream_t st) {
     const long X = Nx + 2, Y = Ny + 2, Z = Nz + 2, XY = X * Y;
     const int nop = r.nop > 0 ? r.nop : 1;
     XLines x{};
-    x.n = Nx; x.nlines = (long)Ny * Nz; x.nA = Ny;
+    if ((long)Ny * Nz > 0x7fffffffL) return hipErrorInvalidValue;
+    x.n = Nx; x.nlines = Ny * Nz; x.nA = Ny;
     x.f = (const z2 *)r.f_e; x.fB = XY * Z; x.fO = XY; x.fC = XY;
     x.out = (z2 *)r.work; x.oB = (long)Nx * Ny * Nz;
     x.lo = (const z2 *)r.fxx_f; x.hi = x.lo + Y * Z; x.eB = 2 * Y * Z; x.e0 = 1 + Y; x.eA = Y;
