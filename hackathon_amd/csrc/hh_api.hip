@@ -1130,7 +1130,15 @@ static void shape_for(int n, long nmodes, int rows, int threads, int wmin, hh::T
 //   complex bands, FP64
 //         n <= 512: 8 rows, 2 rhs, 256 threads: 2D 127: 67 (75), 255: 79
 //         (86), 511: 240 (265); 3D 127^3 x 8: 169 (228);
-//         above: 16 rows, 1 rhs, W >= 4: 2047 x 16: 1292 (1321)
+//         n <= 768: 8 rows, 1 rhs (2 would round differently than a solve of
+//         one), W = 4 up to 800 blocks, 2 from there (k varying with y and
+//         absorbing, against W = 4 with 16 rows): 255 x 520 x 2: 54 (65), x 32:
+//         97 (110), 511 x 640 x 3: 56 (69), x 12: 74 (89), x 64: 355 (431),
+//         400 x 700 x 6, 600 blocks: 60, W = 2: 66 (65), 100 x 700 x 40, 1000
+//         blocks: 67, W = 4: 81 (69);
+//         above: 16 rows, 1 rhs, W >= 4: 2047 x 16: 1292 (1321); 8 rows there
+//         are better and worse by turns: 1023 x 40: 689 (737), 300 x 1000 x 16:
+//         93 (89)
 //   real bands, 2D, FP32 elimination: 16 rows, 512 threads: 1023 x 64:
 //         449 (506), 2047 x 16: 609 (733), 511: 131 (133), 255: 51 (53)
 // and the former rule elsewhere (within 2% of the best shape measured).
@@ -1151,7 +1159,11 @@ static void builtin_tri_shape(const hh_plan *p, bool f32, long per_op, bool real
         else { shape_for(n, nmodes, 16, 256, 1, t); nr = 2; }
     } else if (!f32) {
         if (n <= 512) { shape_for(n, nmodes, 8, 256, 1, t); nr = 2; }
-        else shape_for(n, nmodes, 16, 256, 4, t);
+        else if (n <= 768) {
+            const long blocks = (nmodes + 3) / 4 * p->nop * per_op;
+            const int w = blocks < 800 ? 4 : 2;
+            shape_for(n, nmodes, 8, w * ((n + 7) / 8), w, t);
+        } else shape_for(n, nmodes, 16, 256, 4, t);
     } else if (real && p->dim == 2) {
         shape_for(n, nmodes, 16, 512, 1, t);
     }
