@@ -213,12 +213,11 @@ int hh_plan_flagged_modes(const hh_plan *plan, int op, int *modes, int cap);
  * in {1, 2, 4} right-hand sides of one operator handled together by a
  * thread (the operator's pivots are computed once for them).  Set by the
  * autotuner; (0, 0, *) restores the built-in heuristic.  Shapes differ in
- * speed only: every right-hand side gives the same bits for a given W and
- * rows_per_thread, whatever else is in its batch and whatever rhs_per_thread.
- * get_tri_shape reports the shape a solve uses; for the built-in heuristic
- * it reports rhs_per_thread = 1, though a solve with real bands at 16 rows
- * per thread takes 2 when its batch gives 2048 blocks or more (in mixed
- * precision, when an operator also has two or more right-hand sides). */
+ * speed only: every right-hand side gives the same bits for a given
+ * rows_per_thread, whatever else is in its batch, with complex bands for a
+ * given rhs_per_thread too (rounding alone differs).  get_tri_shape reports
+ * the shape of the solve's elimination (mixed precision: the FP32 one) for a
+ * batch of two right-hand sides per operator. */
 int hh_plan_set_tri_shape(hh_plan *plan, int W, int rows_per_thread, int rhs_per_thread);
 int hh_plan_get_tri_shape(const hh_plan *plan, int *W, int *P, int *rows_per_thread, int *rhs_per_thread);
 /* 2D FFT path: layout of the spectrum between the row DSTs and the mode
@@ -246,7 +245,9 @@ int hh_plan_is_real_operator(const hh_plan *plan);
  * batches of uneven problems, e.g. one plan per grid size.  Solve i runs
  * plans[i] on batch[i] right-hand sides d_rhs[i] -> d_sol[i].  All plans
  * belong to ctx; mixed-precision plans must use fixed sweeps
- * (hh_plan_set_refine(plan, 0, n)).  Tables are built at creation and the
+ * (hh_plan_set_refine(plan, 0, n)).  Solves that share no buffer may run side
+ * by side, in two branches; a result that is another solve's input or result
+ * keeps all of them in the given order.  Tables are built at creation and the
  * graph owns its workspace (freed by hh_graph_destroy), so a launch
  * allocates nothing and later solves on the context do not disturb it; the
  * buffers must stay valid.  Operator values changed by
