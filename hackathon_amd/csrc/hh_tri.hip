@@ -531,7 +531,7 @@ HH_DEV void chain_block(const Prob &prob, const Chains &ch, long block, int batc
     extern __shared__ __align__(16) unsigned char smem_raw[];
     V *carry = reinterpret_cast<V *>(smem_raw);   // C values
     const int n = prob.n(), C = ch.C, PW = 64 / C;   // positions per wave
-    const int NW = ((n + R - 1) / R + PW - 1) / PW;   // waves with rows
+    const int G = (n + R - 1) / R, NW = (G + PW - 1) / PW;   // positions and waves with rows
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     if (wave >= NW && NW == 1) return;   // one wave walks alone, without barriers
     const int c = lane & (C - 1), pw = lane / C;
@@ -577,43 +577,54 @@ HH_DEV void chain_block(const Prob &prob, const Chains &ch, long block, int batc
         Rv[i] = pick(pad, fone, f2);
         Up[i] = pick(pad, fzero, f3);
     }
-    // forward: y_q = d_q - L_q y_{q-1} (L_0 = 0)
+    // forward: y_q = d_q - L_q y_{q-1} (L_0 = 0); backward: x_q = (y_q - Up_q
+    // x_{q+1}) / U_q (2D) or * U_q (3D) (Up_{n-1} = 0).  cnt: the positions of a
+    // wave that hold rows.  A last wave with fewer than PW has loops of its own
+    // (255 x 520: 34 -> 19 us; one loop for both costs the full ones 5%).
     V cy = zero;
+    auto forward = [&](int cnt, bool hand) {
+        for (int pp = 0; pp < cnt; pp++) {
+            if (pw == pp) {
+#pragma unroll
+                for (int i = 0; i < R; i++) {
+                    d[i] = S::fms(L[i], cy, d[i]);
+                    cy = d[i];
+                }
+                if (hand && pp == cnt - 1) carry[c] = cy;
+            }
+            if (pp < cnt - 1) cy = shift(cy, C, true);
+        }
+    };
+    auto backward = [&](int cnt) {
+        for (int pp = cnt - 1; pp >= 0; pp--) {
+            if (pw == pp) {
+#pragma unroll
+                for (int i = R - 1; i >= 0; i--) {
+                    const V a = S::fms(Up[i], cy, d[i]);
+                    if constexpr (Prob::DIM == 2) d[i] = S::div(a, Pv[i], Rv[i]);
+                    else d[i] = S::mul(Rv[i], a);
+                    cy = d[i];
+                }
+                if (pp == 0) carry[c] = cy;
+            }
+            if (pp > 0) cy = shift(cy, C, false);
+        }
+    };
+    const int last = G - (NW - 1) * PW;
     for (int w = 0; w < NW; w++) {
         if (wave == w) {
             if (w > 0) cy = carry[c];
-            for (int pp = 0; pp < PW; pp++) {
-                if (pw == pp) {
-#pragma unroll
-                    for (int i = 0; i < R; i++) {
-                        d[i] = S::fms(L[i], cy, d[i]);
-                        cy = d[i];
-                    }
-                    if (pp == PW - 1) carry[c] = cy;
-                }
-                if (pp < PW - 1) cy = shift(cy, C, true);
-            }
+            if (w == NW - 1 && last < PW) forward(last, false);
+            else forward(PW, true);
         }
         if (NW > 1) __syncthreads();
     }
-    // backward: x_q = (y_q - Up_q x_{q+1}) / U_q (2D) or * U_q (3D) (Up_{n-1} = 0)
     cy = zero;
     for (int w = NW - 1; w >= 0; w--) {
         if (wave == w) {
             if (w < NW - 1) cy = carry[c];
-            for (int pp = PW - 1; pp >= 0; pp--) {
-                if (pw == pp) {
-#pragma unroll
-                    for (int i = R - 1; i >= 0; i--) {
-                        const V a = S::fms(Up[i], cy, d[i]);
-                        if constexpr (Prob::DIM == 2) d[i] = S::div(a, Pv[i], Rv[i]);
-                        else d[i] = S::mul(Rv[i], a);
-                        cy = d[i];
-                    }
-                    if (pp == 0) carry[c] = cy;
-                }
-                if (pp > 0) cy = shift(cy, C, false);
-            }
+            if (w == NW - 1 && last < PW) backward(last);
+            else backward(PW);
         }
         if (NW > 1) __syncthreads();
     }
@@ -650,7 +661,7 @@ template <typename T, int MMAX, class Prob> constexpr int chain_rows() {
 // what it makes of them), so the chains' latency runs beside the elimination
 // instead of before it: one right-hand side at n = 100: 8.3 + 7.4 -> 7.2 us;
 // 6 x 1023^2: 37 + 53 -> 59; 6 x 2047^2: 64 + 263 -> 273; complex, 12 x 511 x 640:
-// 50 + 74 -> 89.
+// 50 + 74 -> 73.
 //
 // Real operators whose table rows are all equal (constant k) take one band per
 // mode, others one per row; which, is read from the device beside the tables,
