@@ -1122,8 +1122,14 @@ static void shape_for(int n, long nmodes, int rows, int threads, int wmin, hh::T
 //   real bands, FP64
 //     2D  n <= 512: 16 rows, 2 rhs, ~512 threads: 127 x 256: 53.9 (60.0),
 //         255 x 64: 59.2 (66.3), 511 x 64: 184 (216);
-//         n <= 1024: 8 rows, 1 rhs, 512 threads: 1023 x 64: 632 (693)
-//         (two blocks of 112 VGPRs per CU against one of 252);
+//         n <= 1024: 16 rows, 2 rhs, W = 4, and 8 above n = 768 from 1024
+//         blocks of 8 on (against 8 rows, 1 rhs, W = 4, one band per mode):
+//         255 x 520 x 1: 19 (24), 1023 x 520 x 40: 152 (263), 511 x 640 x 8:
+//         28 (37), 255 x 768 x 64: 145 (164), 1023 x 850 x 16: 109 (135), 1023
+//         x 1: 37 (44), x 12: 103 (100), x 64: 527 (551), with k varying 601
+//         (769); W = 8 below 1024 blocks or 768 rows: 1023 x 520 x 16: 95 (W =
+//         4: 64), 1023 x 1023 x 6: 60 (51); W = 4 above: 255 x 1000 x 64: 189
+//         (W = 8: 145);
 //         above: 16 rows, 2 rhs, 512 threads: 2047 x 16: 848 (983)
 //     3D  n <= 128: 8 rows, 2 rhs, 128 threads: 127^3 x 8: 138 (147);
 //         above: 16 rows, 256 threads: 255^3 x 1: 187 (212)
@@ -1152,7 +1158,12 @@ static void builtin_tri_shape(const hh_plan *p, bool f32, long per_op, bool real
     int nr = 1;
     if (!f32 && real && p->dim == 2) {
         if (n <= 512) { shape_for(n, nmodes, 16, 512, 1, t); nr = 2; }
-        else if (n <= 1024) shape_for(n, nmodes, 8, 512, 1, t);
+        else if (n <= 1024) {
+            const long blocks = (nmodes + 7) / 8 * p->nop * ((per_op + 1) / 2);
+            const int w = n <= 768 || blocks < 1024 ? 4 : 8;
+            shape_for(n, nmodes, 16, w * ((n + 15) / 16), w, t);
+            nr = 2;
+        }
         else { shape_for(n, nmodes, 16, 512, 1, t); nr = 2; }
     } else if (!f32 && real) {
         if (n <= 128) { shape_for(n, nmodes, 8, 128, 1, t); nr = 2; }
