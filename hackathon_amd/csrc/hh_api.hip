@@ -1131,7 +1131,13 @@ static void shape_for(int n, long nmodes, int rows, int threads, int wmin, hh::T
 //         4: 64), 1023 x 1023 x 6: 60 (51); W = 4 above: 255 x 1000 x 64: 189
 //         (W = 8: 145);
 //         above: 16 rows, 2 rhs, 512 threads: 2047 x 16: 848 (983)
-//     3D  n <= 128: 8 rows, 2 rhs, 128 threads: 127^3 x 8: 138 (147);
+//     3D  n <= 64, or n <= 128 and at most 1024 modes: 8 rows, 2 rhs, 128 threads
+//         (16 rows, W = 8: 20 x 20 x 65 x 2: 10.0 (9.6), 31 x 31 x 65 x 2: 10.2
+//         (10.3), 40 x 40 x 128 x 2: 11.1 (11.4));
+//         n <= 128: 16 rows, 2 rhs, W = 8, and 32 from 1024 blocks of 16 on
+//         (against 8 rows, 128 threads): 52 x 52 x 100: 9.5 (10.3), x 8: 17.5
+//         (21.9), 125^3: 17 (22), x 2: 23 (30), x 4: 43 (49), 127^3 x 8: 99
+//         (124), 255 x 255 x 100: 43 (49); 40 x 40 x 65 x 2: 10.5 (10.2);
 //         above: 16 rows, 256 threads: 255^3 x 1: 187 (212)
 //   complex bands, FP64
 //         n <= 512: 8 rows, 2 rhs, 256 threads: 2D 127: 67 (75), 255: 79
@@ -1156,6 +1162,7 @@ static void builtin_tri_shape(const hh_plan *p, bool f32, long per_op, bool real
     t.nr = 1;
     if (n <= 16) return;
     int nr = 1;
+    const long blocks16 = (nmodes + 15) / 16 * p->nop * ((per_op + 1) / 2);
     if (!f32 && real && p->dim == 2) {
         if (n <= 512) { shape_for(n, nmodes, 16, 512, 1, t); nr = 2; }
         else if (n <= 1024) {
@@ -1166,8 +1173,12 @@ static void builtin_tri_shape(const hh_plan *p, bool f32, long per_op, bool real
         }
         else { shape_for(n, nmodes, 16, 512, 1, t); nr = 2; }
     } else if (!f32 && real) {
-        if (n <= 128) { shape_for(n, nmodes, 8, 128, 1, t); nr = 2; }
-        else { shape_for(n, nmodes, 16, 256, 1, t); nr = 2; }
+        if (n <= 64 || (n <= 128 && nmodes <= 1024)) { shape_for(n, nmodes, 8, 128, 1, t); nr = 2; }
+        else if (n <= 128) {
+            const int w = blocks16 < 1024 ? 8 : 32;
+            shape_for(n, nmodes, 16, w * ((n + 15) / 16), w, t);
+            nr = 2;
+        } else { shape_for(n, nmodes, 16, 256, 1, t); nr = 2; }
     } else if (!f32) {
         if (n <= 512) { shape_for(n, nmodes, 8, 256, 1, t); nr = 2; }
         else if (n <= 768) {
