@@ -162,8 +162,8 @@ struct hh_plan {
     void *d_facc = nullptr, *d_facr = nullptr;
     size_t cap_ent = 0, cap_bits = 0, cap_facc = 0, cap_facr = 0;
     // Generation: bumped whenever a change would invalidate a recorded graph
-    // (device tables reallocated, band kind, operator count or launch shapes
-    // changed); graphs record it at capture and refuse to replay a newer plan.
+    // (device tables reallocated, band kind, operator count, near-resonant mode
+    // counts or launch shapes changed); graphs record it at capture and refuse to replay a newer plan.
     long gen = 0;
 };
 
@@ -1228,10 +1228,11 @@ extern "C" int hh_plan_set_resonance_threshold(hh_plan *p, double kappa) {
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     const int old_nfx = p->ms.nfx;
+    const size_t old_entries = p->ms.fmode.size();   // of all operators: the factors' row length
     p->kappa_flag = kappa;
     hh::classify_modes(p->dim, p->Nx, p->Ny, p->Nz, p->nop, p->hcoef.data(), p->hlamx.data(), p->hlamy.data(),
                        p->real_op != 0, p->kappa_flag, p->ms);
-    if (p->ms.nfx != old_nfx) p->gen++;
+    if (p->ms.nfx != old_nfx || p->ms.fmode.size() != old_entries) p->gen++;
     return upload_tables(p);
 }
 
@@ -1741,8 +1742,9 @@ extern "C" int hh_plan_set_operators(hh_plan *p, int nop, const double *coef) {
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));   // replaced tables may be reallocated
     const int old_real = p->real_op, old_nfx = p->ms.nfx;
+    const size_t old_entries = p->ms.fmode.size();   // of all operators: the factors' row length
     fill_table(p, nop, coef);
-    if (p->real_op != old_real || p->ms.nfx != old_nfx || nop != p->nop) p->gen++;
+    if (p->real_op != old_real || p->ms.nfx != old_nfx || p->ms.fmode.size() != old_entries || nop != p->nop) p->gen++;
     if ((rc = upload_tables(p))) return rc;   // solves queued before this call still read the old ones
     p->nop = nop;
     return HH_OK;
