@@ -1189,8 +1189,12 @@ static void builtin_tri_shape(const hh_plan *p, bool f32, long per_op, bool real
     } else if (real && p->dim == 2) {
         shape_for(n, nmodes, 16, 512, 1, t);
     }
-    const size_t op = real ? 8 : 16;
-    if (nr == 2 && per_op >= 2 && hh::tri_lds_bytes(op, 16, t.P, t.W, 2) <= 160 * 1024) t.nr = 2;
+    // Long complex systems: four modes' reduced systems pass a CU's LDS above
+    // n = 3408 and a block's 1024 threads above 4096 (refused there before); one
+    // mode's fits up to the longest system, 8192 rows (98 KB).
+    const size_t op = (real ? 8 : 16) / (f32 ? 2 : 1), cx = f32 ? 8 : 16, lds = 160 * 1024;
+    while (t.W > 1 && (t.W * t.P > 1024 || hh::tri_lds_bytes(op, cx, t.P, t.W, 1) > lds)) t.W /= 2;
+    if (nr == 2 && per_op >= 2 && hh::tri_lds_bytes(op, cx, t.P, t.W, 2) <= lds) t.nr = 2;
 }
 
 extern "C" int hh_plan_get_tri_shape(const hh_plan *p, int *W, int *P, int *rows_per_thread, int *rhs_per_thread) {
