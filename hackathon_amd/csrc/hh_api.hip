@@ -161,6 +161,10 @@ struct hh_plan {
     uint32_t *d_bits = nullptr;
     void *d_facc = nullptr, *d_facr = nullptr;
     size_t cap_ent = 0, cap_bits = 0, cap_facc = 0, cap_facr = 0;
+    // the operators before the present ones: a replacement that fails goes back to them
+    std::vector<cd> prev_coef;
+    hh::ModeSet prev_ms;
+    int lost = 0;                                // the device tables of neither could be made
     // Generation: bumped whenever a change would invalidate a recorded graph
     // (device tables reallocated, band kind, operator count, near-resonant mode
     // counts or launch shapes changed); graphs record it at capture and refuse to replay a newer plan.
@@ -176,7 +180,10 @@ static int dev_alloc(hh_context *c, void **p, size_t bytes) {
         return fail(HH_ERR_NOMEM, "allocation of %zu bytes exceeds the memory budget (%zu of %zu in use)", bytes,
                     c->in_use, c->budget);
     hipError_t e = hipMalloc(p, bytes ? bytes : 16);
-    if (e != hipSuccess) return fail(HH_ERR_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // a caller that goes on without it must not find the error at its next launch
+        return fail(HH_ERR_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+    }
     c->in_use += bytes;
     return HH_OK;
 }
@@ -762,11 +769,15 @@ static bool table_real(const std::vector<cd> &tab) {
     return true;
 }
 
+static void classify(hh_plan *p, int nop) {
+    hh::classify_modes(p->dim, p->Nx, p->Ny, p->Nz, nop, p->hcoef.data(), p->hlamx.data(), p->hlamy.data(),
+                       p->real_op != 0, p->kappa_flag, p->ms);
+}
+
 static void fill_table(hh_plan *p, int nop, const double *coef) {
     build_table(p->dim, p->dim == 2 ? p->Ny : p->Nz, nop, coef, p->hcoef);
     p->real_op = table_real(p->hcoef);
-    hh::classify_modes(p->dim, p->Nx, p->Ny, p->Nz, nop, p->hcoef.data(), p->hlamx.data(), p->hlamy.data(),
-                       p->real_op != 0, p->kappa_flag, p->ms);
+    classify(p, nop);
 }
 
 // eigenvalues 2cos(k pi/(N+1)), k = 1..N (LU.c:12-14)
@@ -855,6 +866,62 @@ static int upload_tables(hh_plan *p) {
         c->stage_bytes = 0;
     }
     return HH_OK;
+}
+
+// The plan's operators become the nop of coef or, with coef null, are classified
+// again, for the threshold kappa; the context's lock is held.  When the new
+// tables do not fit (memory budget), the plan stays as it was: its mode tables
+// get their old sizes and contents back, after what the new ones took is freed.
+static int replace_operators(hh_plan *p, int nop, const double *coef, double kappa) {
+    hh_context *c = p->ctx;
+    int rc = set_device(c);
+    if (rc) return rc;
+    HIPCHK(hipStreamSynchronize(c->stream));   // replaced tables may be reallocated
+    struct Dev { void **ptr; size_t *cap, was; };
+    Dev dev[4] = {{(void **)&p->d_ent, &p->cap_ent, p->cap_ent}, {(void **)&p->d_bits, &p->cap_bits, p->cap_bits},
+                  {&p->d_facc, &p->cap_facc, p->cap_facc}, {&p->d_facr, &p->cap_facr, p->cap_facr}};
+    const int old_real = p->real_op;
+    const double old_kappa = p->kappa_flag;
+    std::swap(p->ms, p->prev_ms);
+    p->kappa_flag = kappa;
+    if (coef) {
+        p->hcoef.swap(p->prev_coef);
+        fill_table(p, nop, coef);
+    } else {
+        classify(p, nop);
+    }
+    rc = upload_tables(p);   // solves queued before this call still read the old ones
+    if (rc == HH_OK) {
+        const hh::ModeSet &was = p->prev_ms, &now = p->ms;
+        // the sum over all operators is the factors' row length
+        if (p->real_op != old_real || now.nfx != was.nfx || now.fmode.size() != was.fmode.size() || nop != p->nop)
+            p->gen++;
+        p->nop = nop;
+        p->lost = 0;
+        if (was.facr.size() + 2 * was.facc.size() > ((size_t)1 << 20)) p->prev_ms = hh::ModeSet();   // 8 MiB
+        return HH_OK;
+    }
+    const std::string why = g_err;
+    std::swap(p->ms, p->prev_ms);
+    if (coef) p->hcoef.swap(p->prev_coef);
+    p->real_op = old_real;
+    p->kappa_flag = old_kappa;
+    for (Dev &d : dev)
+        if (*d.ptr && *d.cap != d.was) {
+            dev_free(c, *d.ptr, *d.cap);
+            *d.ptr = nullptr;
+            *d.cap = 0;
+        }
+    int back = HH_OK;
+    for (Dev &d : dev)
+        if (back == HH_OK) back = ensure_dev(p, d.ptr, d.cap, d.was);
+    if (back == HH_OK) back = upload_tables(p);
+    if (back != HH_OK) {
+        p->lost = 1;
+        p->gen++;
+    }
+    g_err = why;
+    return rc;
 }
 
 static int upload_plan(hh_plan *p, int ncoef, int n) {
@@ -1226,18 +1293,8 @@ extern "C" int hh_plan_get_tri_shape(const hh_plan *p, int *W, int *P, int *rows
 
 extern "C" int hh_plan_set_resonance_threshold(hh_plan *p, double kappa) {
     if (!p || !(kappa >= 0)) return fail(HH_ERR_ARG, "hh_plan_set_resonance_threshold: bad arguments");
-    hh_context *c = p->ctx;
-    std::lock_guard<std::mutex> lk(c->mu);
-    int rc = set_device(c);
-    if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(c->stream));
-    const int old_nfx = p->ms.nfx;
-    const size_t old_entries = p->ms.fmode.size();   // of all operators: the factors' row length
-    p->kappa_flag = kappa;
-    hh::classify_modes(p->dim, p->Nx, p->Ny, p->Nz, p->nop, p->hcoef.data(), p->hlamx.data(), p->hlamy.data(),
-                       p->real_op != 0, p->kappa_flag, p->ms);
-    if (p->ms.nfx != old_nfx || p->ms.fmode.size() != old_entries) p->gen++;
-    return upload_tables(p);
+    std::lock_guard<std::mutex> lk(p->ctx->mu);
+    return replace_operators(p, p->nop, nullptr, kappa);
 }
 
 extern "C" int hh_plan_mode_info(const hh_plan *p, int op, int *flagged, int *singular, double *kappa) {
@@ -1419,8 +1476,10 @@ static int norms_sync(hh_context *c, long n, const void *x, const void *y, doubl
 }
 
 // HH_ERR_SINGULAR when an operator that right-hand sides 0..batch-1 use is
-// singular to working precision.
-static int check_singular(const hh_plan *p, int batch) {
+// singular to working precision; HH_ERR_NOMEM when a failed replacement of the
+// operators left the plan without device tables.
+static int check_operators(const hh_plan *p, int batch) {
+    if (p->lost) return fail(HH_ERR_NOMEM, "the plan lost its operators' tables when replacing them failed; set them again");
     const int used = batch < p->nop ? batch : p->nop;
     for (int o = 0; o < used; o++)
         if (p->ms.singular[o])
@@ -1483,7 +1542,7 @@ static int solve_ws(hh_plan *p, const void *rhs, void *sol, int batch, void *scr
 
 static int solve_locked(hh_plan *p, const void *rhs, void *sol, int batch) {
     hh_context *c = p->ctx;
-    int rc = check_singular(p, batch);
+    int rc = check_operators(p, batch);
     if (rc) return rc;
     if ((rc = set_device(c))) return rc;
     size_t ws_bytes = hh_plan_workspace_bytes(p, batch);
@@ -1498,6 +1557,7 @@ int hh::solve_one(hh_plan *p, int op, const void *rhs, void *sol) {
         return fail(HH_ERR_ARG, "internal: bad single solve");
     hh_context *c = p->ctx;
     std::lock_guard<std::mutex> lk(c->mu);
+    if (p->lost) return check_operators(p, 1);
     if (p->ms.singular[op]) return fail(HH_ERR_SINGULAR, "operator %d is singular to working precision", op);
     int rc = set_device(c);
     if (rc) return rc;
@@ -1512,7 +1572,7 @@ extern "C" int hh_solve_noalloc(hh_plan *p, const void *rhs, void *sol, int batc
     if (batch < 1) return fail(HH_ERR_ARG, "hh_solve_noalloc: batch must be >= 1 (got %d)", batch);
     hh_context *c = p->ctx;
     std::lock_guard<std::mutex> lk(c->mu);
-    int rc = check_singular(p, batch);
+    int rc = check_operators(p, batch);
     if (rc) return rc;
     if ((rc = set_device(c))) return rc;
     if (!c->noalloc_ws)
@@ -1618,7 +1678,7 @@ extern "C" int hh_graph_create(hh_context *c, int nsolves, hh_plan *const *plans
         if (p->prec == HH_PREC_MIXED && p->tol != 0)
             return fail(HH_ERR_UNSUPPORTED, "hh_graph_create: mixed-precision plan %d needs fixed sweeps "
                                             "(hh_plan_set_refine(plan, 0, sweeps))", i);
-        if ((rc = check_singular(p, batch[i]))) return rc;
+        if ((rc = check_operators(p, batch[i]))) return rc;
         if ((rc = prepare_tables(p))) return rc;
     }
     std::vector<int> branch = graph_branches(nsolves, plans, d_rhs, d_sol, batch);
@@ -1740,18 +1800,8 @@ extern "C" int hh_plan_set_operators(hh_plan *p, int nop, const double *coef) {
     if (!p || !coef) return fail(HH_ERR_ARG, "hh_plan_set_operators: null argument");
     if (nop < 1 || nop > p->cap_nop)
         return fail(HH_ERR_ARG, "hh_plan_set_operators: %d operators, the plan holds at most %d", nop, p->cap_nop);
-    hh_context *c = p->ctx;
-    std::lock_guard<std::mutex> lk(c->mu);
-    int rc = set_device(c);
-    if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(c->stream));   // replaced tables may be reallocated
-    const int old_real = p->real_op, old_nfx = p->ms.nfx;
-    const size_t old_entries = p->ms.fmode.size();   // of all operators: the factors' row length
-    fill_table(p, nop, coef);
-    if (p->real_op != old_real || p->ms.nfx != old_nfx || p->ms.fmode.size() != old_entries || nop != p->nop) p->gen++;
-    if ((rc = upload_tables(p))) return rc;   // solves queued before this call still read the old ones
-    p->nop = nop;
-    return HH_OK;
+    std::lock_guard<std::mutex> lk(p->ctx->mu);
+    return replace_operators(p, nop, coef, p->kappa_flag);
 }
 
 extern "C" int hh_solve_host(hh_plan *p, const double *h_rhs, double *h_sol, int batch) {

@@ -171,7 +171,9 @@ int hh_plan_last_refine(const hh_plan *plan, int *sweeps, double *rel_residual);
  * 1 <= nop <= the count it was created with (no reference counterpart: lets
  * a serving loop reuse one device-resident plan per grid for every batch).
  * coef has the layout of the create_multi call.  Waits for the work already
- * queued on the context's stream, then queues the new tables on it. */
+ * queued on the context's stream, then queues the new tables on it.  When
+ * they do not fit the memory budget (HH_ERR_NOMEM) the plan keeps the
+ * operators it has; hh_plan_set_resonance_threshold likewise. */
 int hh_plan_set_operators(hh_plan *plan, int nop, const double *coef);
 /* Near-resonant modes (no reference counterpart; the reference's LU() divides
  * by whatever pivot it meets, 2D_Program/main_functions/LU.c:36,
