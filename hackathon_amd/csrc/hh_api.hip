@@ -1636,9 +1636,19 @@ static int prepare_tables(hh_plan *p) {
 // launches and latencies of small grids lie beside a large one's memory
 // traffic: each solve goes to the branch with less work so far, largest
 // first.  63 .. 2047 squared x 6: 890 -> 810 us; 300, 511, 1023 squared x 2: 160 ->
-// 111; two solves whose lighter one is short lose (63, 100 squared: 36 -> 44;
-// 255, 300 squared x 3, 3 MB: 68 and 67) and keep one branch.  As soon as one
-// solve's result is another's input or result, all keep the caller's order on one branch.
+// 111.  As soon as one solve's result is another's input or result, all keep the
+// caller's order on one branch.
+//
+// Short lists keep one branch too.  Two solves whose lighter one is short lose
+// (63, 100 squared: 36 -> 44; 255, 300 squared x 3, 3 MB: 68 and 67).  Of three
+// and more, one branch takes about 15 us a solve and 3.5 us a MB, two take at
+// least 45 us and 9 a solve, whatever its size; the line lies where these meet.
+// Below it, one and two branches: 3 x 63 squared 54 and 69 to 76 us; 40, 63, 100
+// squared 47 and 74; 5 x 63 squared 86 and 100; 4 x 100 squared x 8 71 and 79;
+// 3 x 255 squared 68 and 72.  Above: 8 x 127 squared 148 and 125; 3 x 300 squared
+// x 2 95 and 77; 80, 255, 640 squared 106 and 81.  Of 130 lists two were up to 14
+// us slower than one above the line (6 x 100 squared x 2) and up to 10 us faster
+// below it (6 x 127 squared).
 static std::vector<int> graph_branches(int nsolves, hh_plan *const *plans, void *const *d_rhs, void *const *d_sol,
                                        const int *batch) {
     std::vector<int> branch(nsolves, 0);
@@ -1659,7 +1669,9 @@ static std::vector<int> graph_branches(int nsolves, hh_plan *const *plans, void 
         branch[i] = load[1] < load[0];
         load[branch[i]] += bytes[i];
     }
-    if (nsolves == 2 && load[1] < ((size_t)4 << 20)) branch.assign(2, 0);
+    const size_t mib = (size_t)1 << 20;
+    const bool few = nsolves == 2 ? load[1] < 4 * mib : load[0] + load[1] + nsolves * (mib + 3 * mib / 4) < 12 * mib;
+    if (few) branch.assign(nsolves, 0);
     return branch;
 }
 
