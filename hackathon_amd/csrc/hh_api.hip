@@ -1649,8 +1649,10 @@ static int prepare_tables(hh_plan *p) {
 // x 2 95 and 77; 80, 255, 640 squared 106 and 81.  Of 130 lists two were up to 14
 // us slower than one above the line (6 x 100 squared x 2) and up to 10 us faster
 // below it (6 x 127 squared).
+//
+// one_workspace: every solve that needs one on the same branch.
 static std::vector<int> graph_branches(int nsolves, hh_plan *const *plans, void *const *d_rhs, void *const *d_sol,
-                                       const int *batch) {
+                                       const int *batch, bool one_workspace) {
     std::vector<int> branch(nsolves, 0);
     std::vector<size_t> bytes(nsolves);
     for (int i = 0; i < nsolves; i++) bytes[i] = (size_t)hh_plan_field_size(plans[i]) * batch[i] * 16;
@@ -1665,12 +1667,16 @@ static std::vector<int> graph_branches(int nsolves, hh_plan *const *plans, void 
     for (int i = 0; i < nsolves; i++) by[i] = i;
     std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return bytes[a] > bytes[b]; });
     size_t load[2] = {0, 0};
+    auto bound = [&](int i) { return one_workspace && hh_plan_workspace_bytes(plans[i], batch[i]) > 0; };
+    for (int i : by)
+        if (bound(i)) load[0] += bytes[i];
     for (int i : by) {
+        if (bound(i)) continue;
         branch[i] = load[1] < load[0];
         load[branch[i]] += bytes[i];
     }
     const size_t mib = (size_t)1 << 20;
-    const bool few = nsolves == 2 ? load[1] < 4 * mib : load[0] + load[1] + nsolves * (mib + 3 * mib / 4) < 12 * mib;
+    const bool few = nsolves == 2 ? std::min(load[0], load[1]) < 4 * mib : load[0] + load[1] + nsolves * (mib + 3 * mib / 4) < 12 * mib;
     if (few) branch.assign(nsolves, 0);
     return branch;
 }
@@ -1693,11 +1699,14 @@ extern "C" int hh_graph_create(hh_context *c, int nsolves, hh_plan *const *plans
         if ((rc = check_operators(p, batch[i]))) return rc;
         if ((rc = prepare_tables(p))) return rc;
     }
-    std::vector<int> branch = graph_branches(nsolves, plans, d_rhs, d_sol, batch);
+    // Under a memory budget a graph takes no more than its solves would one after
+    // the other: what a second workspace took would be refused to a later solve.
+    std::vector<int> branch = graph_branches(nsolves, plans, d_rhs, d_sol, batch, c->budget > 0);
     auto workspace = [&]() {
         part[0] = part[1] = 0;
         for (int i = 0; i < nsolves; i++)
-            part[branch[i]] = std::max(part[branch[i]], (hh_plan_workspace_bytes(plans[i], batch[i]) + 255) & ~(size_t)255);
+            part[branch[i]] = std::max(part[branch[i]], hh_plan_workspace_bytes(plans[i], batch[i]));
+        if (part[1] > 0) part[0] = (part[0] + 255) & ~(size_t)255;
         return part[0] + part[1];
     };
     size_t ws = workspace();

@@ -249,7 +249,8 @@ int hh_plan_is_real_operator(const hh_plan *plan);
  * belong to ctx; mixed-precision plans must use fixed sweeps
  * (hh_plan_set_refine(plan, 0, n)).  Solves that share no buffer may run side
  * by side, in two branches; a result that is another solve's input or result
- * keeps all of them in the given order.  Tables are built at creation and the
+ * keeps all of them in the given order.  With a memory budget set the graph's
+ * workspace is that of its largest solve, else up to one per branch.  Tables are built at creation and the
  * graph owns its workspace (freed by hh_graph_destroy), so a launch
  * allocates nothing and later solves on the context do not disturb it; the
  * buffers must stay valid.  Operator values changed by
