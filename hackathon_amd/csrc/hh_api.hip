@@ -55,6 +55,8 @@ static int fail(int code, const char *fmt, ...) {
                         __FILE__, __LINE__);                                                       \
     } while (0)
 
+constexpr size_t STAGE_LEAST = (size_t)256 << 10, STAGE_MOST = (size_t)8 << 20;
+
 struct hh_context {
     int device = 0;
     hipStream_t own = nullptr, stream = nullptr;
@@ -68,8 +70,8 @@ struct hh_context {
     // their two results, in host memory that the kernels write (copied from the
     // device they cost a refinement 28 us more per sweep)
     double *h_norm = nullptr;
-    // pinned memory from which the device reads a plan's operator tables, and
-    // the event of its last reader
+    // pinned memory from which the device reads a plan's operator tables (from
+    // STAGE_LEAST up to STAGE_MOST), and the event of its last reader
     void *stage = nullptr;
     size_t stage_bytes = 0;
     hipEvent_t staged = nullptr;
@@ -441,13 +443,16 @@ extern "C" int hh_context_create(int device, hh_context **out) {
     if (hipMalloc((void **)&c->d_norm, 2 * (hh::NORM_BLOCKS + hh::NORM_SLOTS) * sizeof(double)) != hipSuccess ||
         hipMemcpy(c->residual_slots(), zeros.data(), zeros.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
         hipHostMalloc((void **)&c->h_norm, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(&c->stage, STAGE_LEAST, hipHostMallocDefault) != hipSuccess ||
         hipEventCreateWithFlags(&c->staged, hipEventDisableTiming) != hipSuccess) {
+        (void)hipHostFree(c->stage);
         (void)hipHostFree(c->h_norm);
         (void)hipFree(c->d_norm);
         (void)hipStreamDestroy(c->own);
         delete c;
         return fail(HH_ERR_NOMEM, "norm buffer allocation failed");
     }
+    c->stage_bytes = STAGE_LEAST;
     *out = c;
     return HH_OK;
 }
@@ -810,6 +815,23 @@ static int ensure_dev(hh_plan *p, void **ptr, size_t *cap, size_t bytes) {
     return HH_OK;
 }
 
+// Staging memory for `bytes`, up to STAGE_MOST: pinning is slow (94 MiB for the
+// factors of every mode of 127^3: 20 ms of 45, in pieces 25).  The one there
+// stays where a larger one cannot be had.
+static void grow_stage(hh_context *c, size_t bytes) {
+    if (bytes <= c->stage_bytes || c->stage_bytes >= STAGE_MOST) return;
+    const size_t want = std::min((bytes + bytes / 2 + 15) / 16 * 16, STAGE_MOST);
+    void *more = nullptr;
+    if (hipHostMalloc(&more, want, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    (void)hipEventSynchronize(c->staged);
+    (void)hipHostFree(c->stage);
+    c->stage = more;
+    c->stage_bytes = want;
+}
+
 // The device tables of the plan's operators (nop of them in hcoef and ms) from
 // the host's, stream-ordered after the work already queued; the context's lock
 // is held.
@@ -826,44 +848,44 @@ static int upload_tables(hh_plan *p) {
     if ((rc = ensure_dev(p, (void **)&p->d_bits, &p->cap_bits, m.bits.size() * sizeof(uint32_t)))) return rc;
     if ((rc = ensure_dev(p, &p->d_facc, &p->cap_facc, nf * sizeof(cd)))) return rc;
     if ((rc = ensure_dev(p, &p->d_facr, &p->cap_facr, (p->real_op ? nf : 0) * sizeof(double)))) return rc;
-    // staging: bands, factors, entries, bits (each a multiple of 16 bytes)
+    // bands, factors, entries and bits go through the staging memory in turn, as
+    // much at a time as it holds
+    const size_t fac = p->real_op ? sizeof(double) : sizeof(cd), unit[4] = {sizeof(cd), fac, sizeof(int2), sizeof(uint32_t)};
     const void *src[4] = {p->hcoef.data(), p->real_op ? (const void *)m.facr.data() : (const void *)m.facc.data(),
                           p->hent.data(), m.bits.data()};
-    const size_t len[4] = {p->hcoef.size() * sizeof(cd), nf * (p->real_op ? sizeof(double) : sizeof(cd)),
-                           p->hent.size() * sizeof(int2), m.bits.size() * sizeof(uint32_t)};
-    size_t at[4], total = 0;
-    for (int k = 0; k < 4; k++) { at[k] = total; total += (len[k] + 15) / 16 * 16; }
-    HIPCHK(hipEventSynchronize(c->staged));
-    if (total > c->stage_bytes) {
-        const size_t want = std::max(total + total / 2, (size_t)256 << 10);
-        (void)hipHostFree(c->stage);
-        c->stage = nullptr;
-        c->stage_bytes = 0;
-        if (hipHostMalloc(&c->stage, want, hipHostMallocDefault) != hipSuccess)
-            return fail(HH_ERR_NOMEM, "pinned allocation of %zu bytes failed", want);
-        c->stage_bytes = want;
-    }
-    char *base = (char *)c->stage;
-    for (int k = 0; k < 4; k++)
-        if (len[k]) memcpy(base + at[k], src[k], len[k]);
-    hh::OperatorTables t;
-    t.ncoef = (long)p->hcoef.size();
-    t.coef = (const double2 *)(base + at[0]);
-    t.coef64 = (double2 *)p->coef64; t.coef32 = (float2 *)p->coef32;
-    t.coefr64 = (double *)p->coefr64; t.coefr32 = (float *)p->coefr32;
-    t.n = m.n; t.nent = (long)ne;
-    (p->real_op ? (const void *&)t.facr : (const void *&)t.facc) = base + at[1];
-    t.outr = (double *)p->d_facr; t.outc = (double2 *)p->d_facc;
-    t.nslot = (long)p->hent.size(); t.ent = (const int2 *)(base + at[2]); t.outent = p->d_ent;
-    t.nbits = (long)m.bits.size(); t.bits = (const uint32_t *)(base + at[3]); t.outbits = p->d_bits;
-    const hipError_t e = hh::launch_operator_tables(t, c->stream);
-    if (e != hipSuccess) return fail(HH_ERR_DEVICE, "operator tables: launch failed: %s", hipGetErrorString(e));
-    HIPCHK(hipEventRecord(c->staged, c->stream));
-    if (c->stage_bytes > ((size_t)8 << 20)) {   // kept for the next operators only while it is small
+    const size_t len[4] = {p->hcoef.size(), nf, p->hent.size(), m.bits.size()};
+    size_t total = 0, done[4] = {};
+    for (int k = 0; k < 4; k++) total += (len[k] * unit[k] + 15) / 16 * 16;
+    grow_stage(c, total);
+    for (bool more = true; more;) {
         HIPCHK(hipEventSynchronize(c->staged));
-        (void)hipHostFree(c->stage);
-        c->stage = nullptr;
-        c->stage_bytes = 0;
+        size_t at[4], n[4], used = 0;
+        for (int k = 0; k < 4; k++) {
+            at[k] = used;
+            n[k] = std::min(len[k] - done[k], (c->stage_bytes - used) / unit[k]);
+            if (n[k]) memcpy((char *)c->stage + used, (const char *)src[k] + done[k] * unit[k], n[k] * unit[k]);
+            used += (n[k] * unit[k] + 15) / 16 * 16;
+        }
+        const char *base = (const char *)c->stage;
+        hh::OperatorTables t;
+        t.ncoef = (long)n[0];
+        t.coef = (const double2 *)(base + at[0]);
+        t.coef64 = (double2 *)p->coef64 + done[0]; t.coef32 = (float2 *)p->coef32 + done[0];
+        t.coefr64 = (double *)p->coefr64 + done[0]; t.coefr32 = (float *)p->coefr32 + done[0];
+        t.n = m.n; t.nent = (long)ne;
+        t.fac0 = (long)done[1]; t.nfac = (long)n[1];
+        (p->real_op ? (const void *&)t.facr : (const void *&)t.facc) = base + at[1];
+        t.outr = (double *)p->d_facr; t.outc = (double2 *)p->d_facc;
+        t.nslot = (long)n[2]; t.ent = (const int2 *)(base + at[2]); t.outent = p->d_ent + done[2];
+        t.nbits = (long)n[3]; t.bits = (const uint32_t *)(base + at[3]); t.outbits = p->d_bits + done[3];
+        const hipError_t e = hh::launch_operator_tables(t, c->stream);
+        if (e != hipSuccess) return fail(HH_ERR_DEVICE, "operator tables: launch failed: %s", hipGetErrorString(e));
+        HIPCHK(hipEventRecord(c->staged, c->stream));
+        more = false;
+        for (int k = 0; k < 4; k++) {
+            done[k] += n[k];
+            more = more || done[k] < len[k];
+        }
     }
     return HH_OK;
 }

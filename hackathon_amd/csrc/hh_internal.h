@@ -114,7 +114,7 @@ struct ModeSet {
 void classify_modes(int dim, int Nx, int Ny, int Nz, int nop, const std::complex<double> *hcoef,
                     const double *lamx, const double *lamy, bool real, double kappa_flag, ModeSet &ms);
 
-// Sources (host-accessible or device memory) and device tables of a plan's operators.
+// Sources (host-accessible or device memory) and device tables of a plan's operators, or a part of them.
 struct OperatorTables {
     long ncoef = 0;                       // band table
     const double2 *coef = nullptr;
@@ -123,6 +123,7 @@ struct OperatorTables {
     double *coefr64 = nullptr;
     float *coefr32 = nullptr;
     long n = 0, nent = 0;                 // factors: rows, entries; facr where they are real, else facc
+    long fac0 = 0, nfac = 0;              // first value here and how many
     const double *facr = nullptr;
     const double2 *facc = nullptr;
     double *outr = nullptr;

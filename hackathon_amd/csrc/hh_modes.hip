@@ -348,8 +348,8 @@ __global__ __launch_bounds__(256) void k_operator_tables(OperatorTables t) {
         t.coefr32[i] = (float)v.x;
     }
     const long per = 4L * t.n;   // values of one entry
-    for (long i = id; i < t.nent * per; i += step) {
-        const long e = i / per, r = i - e * per, q = r >> 2, to = (q * t.nent + e) * 4 + (r & 3);
+    for (long i = id; i < t.nfac; i += step) {
+        const long g = t.fac0 + i, e = g / per, r = g - e * per, q = r >> 2, to = (q * t.nent + e) * 4 + (r & 3);
         if (t.facr) {
             const double v = t.facr[i];
             t.outr[to] = v;
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(256) void k_operator_tables(OperatorTables t) {
 }
 
 hipError_t launch_operator_tables(const OperatorTables &t, hipStream_t st) {
-    const long work = std::max(std::max(t.ncoef, 4 * t.nent * t.n), std::max(t.nslot, t.nbits));
+    const long work = std::max(std::max(t.ncoef, t.nfac), std::max(t.nslot, t.nbits));
     const long blocks = std::min(1024L, (work + 255) / 256);
     hipLaunchKernelGGL(k_operator_tables, dim3((unsigned)std::max(1L, blocks)), dim3(256), 0, st, t);
     return hipGetLastError();
