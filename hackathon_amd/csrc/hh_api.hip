@@ -484,7 +484,25 @@ extern "C" int hh_context_set_stream(hh_context *c, void *stream) {
     if (!c) return fail(HH_ERR_ARG, "null context");
     // NULL is the HIP default (null) stream, which orders against the work
     // of callers (e.g. PyTorch's default stream) that use it
-    c->stream = (hipStream_t)stream;
+    const hipStream_t next = (hipStream_t)stream;
+    if (next == c->stream) return HH_OK;
+    // Replaced operators' tables may still be on their way on the stream before:
+    // the next one waits for them, or the host where it is being recorded (a
+    // wait for work outside it would end the recording).
+    int rc = set_device(c);
+    if (rc) return rc;
+    hipStreamCaptureStatus recording = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(next, &recording) == hipSuccess && recording == hipStreamCaptureStatusNone) {
+        HIPCHK(hipStreamWaitEvent(next, c->staged, 0));
+    } else {
+        (void)hipGetLastError();
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        HIPCHK(hipThreadExchangeStreamCaptureMode(&mode));
+        const hipError_t e = hipEventSynchronize(c->staged);
+        HIPCHK(hipThreadExchangeStreamCaptureMode(&mode));
+        HIPCHK(e);
+    }
+    c->stream = next;
     return HH_OK;
 }
 

@@ -44,7 +44,9 @@ const char *hh_status_string(int status);
 int hh_context_create(int device, hh_context **ctx);
 int hh_context_destroy(hh_context *ctx);
 /* run on a caller stream (hipStream_t); NULL selects the HIP default (null)
- * stream.  A new context runs on a private non-blocking stream. */
+ * stream.  A new context runs on a private non-blocking stream.  Operators
+ * that were replaced on the stream before are complete for work on the new
+ * one; other work of the two is ordered by the caller. */
 int hh_context_set_stream(hh_context *ctx, void *stream);
 void *hh_context_get_stream(hh_context *ctx);
 int hh_context_synchronize(hh_context *ctx);
