@@ -443,16 +443,13 @@ extern "C" int hh_context_create(int device, hh_context **out) {
     if (hipMalloc((void **)&c->d_norm, 2 * (hh::NORM_BLOCKS + hh::NORM_SLOTS) * sizeof(double)) != hipSuccess ||
         hipMemcpy(c->residual_slots(), zeros.data(), zeros.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
         hipHostMalloc((void **)&c->h_norm, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc(&c->stage, STAGE_LEAST, hipHostMallocDefault) != hipSuccess ||
         hipEventCreateWithFlags(&c->staged, hipEventDisableTiming) != hipSuccess) {
-        (void)hipHostFree(c->stage);
         (void)hipHostFree(c->h_norm);
         (void)hipFree(c->d_norm);
         (void)hipStreamDestroy(c->own);
         delete c;
         return fail(HH_ERR_NOMEM, "norm buffer allocation failed");
     }
-    c->stage_bytes = STAGE_LEAST;
     *out = c;
     return HH_OK;
 }
@@ -834,20 +831,23 @@ static int ensure_dev(hh_plan *p, void **ptr, size_t *cap, size_t bytes) {
 }
 
 // Staging memory for `bytes`, up to STAGE_MOST: pinning is slow (94 MiB for the
-// factors of every mode of 127^3: 20 ms of 45, in pieces 25).  The one there
-// stays where a larger one cannot be had.
-static void grow_stage(hh_context *c, size_t bytes) {
-    if (bytes <= c->stage_bytes || c->stage_bytes >= STAGE_MOST) return;
-    const size_t want = std::min((bytes + bytes / 2 + 15) / 16 * 16, STAGE_MOST);
+// factors of every mode of 127^3: 20 ms of 45, in pieces 25).  Where that much
+// cannot be had, the one there stays or a smaller one does.
+static int grow_stage(hh_context *c, size_t bytes) {
+    if (bytes <= c->stage_bytes || c->stage_bytes >= STAGE_MOST) return HH_OK;
+    size_t want = std::min(std::max((bytes + bytes / 2 + 15) / 16 * 16, STAGE_LEAST), STAGE_MOST);
     void *more = nullptr;
-    if (hipHostMalloc(&more, want, hipHostMallocDefault) != hipSuccess) {
+    while (hipHostMalloc(&more, want, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
-        return;
+        if (c->stage) return HH_OK;
+        if (want <= 4096) return fail(HH_ERR_NOMEM, "pinned allocation of %zu bytes failed", want);
+        want = want / 32 * 16;
     }
     (void)hipEventSynchronize(c->staged);
     (void)hipHostFree(c->stage);
     c->stage = more;
     c->stage_bytes = want;
+    return HH_OK;
 }
 
 // The device tables of the plan's operators (nop of them in hcoef and ms) from
@@ -874,7 +874,7 @@ static int upload_tables(hh_plan *p) {
     const size_t len[4] = {p->hcoef.size(), nf, p->hent.size(), m.bits.size()};
     size_t total = 0, done[4] = {};
     for (int k = 0; k < 4; k++) total += (len[k] * unit[k] + 15) / 16 * 16;
-    grow_stage(c, total);
+    if ((rc = grow_stage(c, total))) return rc;
     for (bool more = true; more;) {
         HIPCHK(hipEventSynchronize(c->staged));
         size_t at[4], n[4], used = 0;
@@ -1207,8 +1207,8 @@ extern "C" int hh_plan_set_tile_width(hh_plan *p, int tw) {
 }
 
 // Shape of `rows` rows per thread and about `threads` threads per block:
-// W the largest power of two with W P <= threads, in [wmin, 16], and no
-// more than the modes need.
+// W the largest power of two with W P <= threads, up to 16 (at least wmin,
+// which may be more), and no more than the modes need.
 static void shape_for(int n, long nmodes, int rows, int threads, int wmin, hh::TriHelm &t) {
     int P = (n + rows - 1) / rows;
     if (P > n / 2) P = n / 2;
