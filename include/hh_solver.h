@@ -290,7 +290,8 @@ int hh_dst2d_layers(hh_context *ctx, int Nx, int Ny, long nlayers, const void *d
  * ghost ring: bottom row, top row, left column, right column
  * (2(Nx+2)+2(Ny+2)).  Host, complex: k2e = k^2 at y0 + j*hy (Ny+2), k2yb =
  * (k^2)_y at y0, y1 (2), each repeated per operator of a multi-operator
- * plan.  Orders 2 and 4 ignore fy_b, fxx_b, fyy_b, k2yb. */
+ * plan.  Orders 2 and 4 ignore fy_b, fxx_b, fyy_b, k2yb.  Order 6 takes lines
+ * of up to 16384 points (Nx here, Nx and Ny in 3D; a launch error above). */
 int hh_rhs2d(hh_plan *plan, int order, double hx, double hy, const void *d_f_e, const void *d_u_e,
              const void *d_fy_b, const void *d_fxx_b, const void *d_fyy_b, const double *k2e,
              const double *k2yb, void *d_F, int batch);
